@@ -28,14 +28,12 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path[:0] = [os.path.join(ROOT, "solstice-solver_amd", "python")]
 
 HBM_PEAK_GBS = 8000.0
-# Algorithmic bytes per traced segment (FP64 path state):
-#  trace kernel: reads the 56 B of path state it needs, writes a 32 B hit record
-#  shade kernel: reads path state (96 B) and hit (32 B), writes path state
-#                (96 B) and the compacted queue index (8 B)
-BYTES_TRACE_FP64 = 56 + 32
-BYTES_SHADE_FP64 = 96 + 32 + 96 + 8
-BYTES_TRACE_FP32 = 40 + 16
-BYTES_SHADE_FP32 = 64 + 16 + 64 + 8
+# Algorithmic bytes per traced segment of the path kernels (k_start and
+# k_resume, which trace a ray and shade its hit): the path's record is read
+# and written (176 B in FP64, 112 B in FP32) through a 4 B list entry, itself
+# written and read
+BYTES_PATH_FP64 = 176 + 176 + 8
+BYTES_PATH_FP32 = 112 + 112 + 8
 
 # Work started within a few seconds of closing a context that held tens of
 # GB of device memory ran up to 2x slower on MI355X (the kernels' own times
@@ -408,21 +406,12 @@ def main(argv=None):
     value = args.steps * B / total / 1e6
     g = est.global_()
 
-    # roofline of the dominant kernel, from in-stream HIP events (the
-    # host-driven loop records them; a graph-captured run has none)
+    # roofline of the path kernels, from in-stream HIP events
     fp32 = args.precision == "fp32"
-    if trace_ms <= 0 and shade_ms <= 0:
-        print("bench.py: no per-kernel times (graph mode); run with --graph 0 for the roofline",
-              file=sys.stderr)
-        trace_ms = shade_ms = float("nan")
-    if not (shade_ms > trace_ms):
-        kernel, ms, per_seg = "k_trace", trace_ms, (BYTES_TRACE_FP32 if fp32 else BYTES_TRACE_FP64)
-    else:
-        kernel, ms, per_seg = "k_shade", shade_ms, (BYTES_SHADE_FP32 if fp32 else BYTES_SHADE_FP64)
+    kernel, ms = ("k_path32" if fp32 else "k_path"), trace_ms
+    per_seg = BYTES_PATH_FP32 if fp32 else BYTES_PATH_FP64
     achieved = per_seg * segs / (ms * 1e-3) / 1e9
     seg_per_launch = segs / iters
-    if fp32:
-        kernel += "32"   # the FP32 form's kernels: k_trace32, k_shade32
     tr = load_traffic(kernel, workload + ("_fp32" if fp32 else ""))
     traffic = None if tr is None else round(tr["hbm_bytes_per_segment"] * seg_per_launch)
     roofline = {"bound": "hbm", "kernel": kernel, "achieved": round(achieved, 2),

@@ -641,9 +641,9 @@ struct ssol_solve_stats {
   uint64_t paths;
   uint64_t pending_spills; /* per-path pending tally entries flushed early */
   double kernel_ms;
-  double trace_ms;
-  double shade_ms;
-  unsigned iterations;
+  double trace_ms;         /* of these, the path kernels (trace and shade in one) */
+  double shade_ms;         /* 0: shading has no kernel of its own */
+  unsigned iterations;     /* generations of rays, the most any path had */
   unsigned wavefronts; /* wavefronts started: chunks of realisations all in
                           flight (a narrow width), or 1 */
   unsigned refilled;   /* 1: slots took further realisations in place */
@@ -651,8 +651,8 @@ struct ssol_solve_stats {
 SSOL_API res_T ssol_estimator_get_solve_stats
   (const struct ssol_estimator* estimator, struct ssol_solve_stats* stats);
 
-/* Wavefront iterations captured per HIP graph launch (0, the default: one
- * host round trip per iteration). */
+/* Kept for programs that set it: solves launch one kernel per generation of
+ * rays, and one for the last few paths, whatever the value. */
 SSOL_API res_T ssol_device_set_graph_iterations
   (struct ssol_device* dev, const unsigned iterations);
 

@@ -271,9 +271,9 @@ struct ssolh_solve_args {
   uint32_t precision;         /* enum ssolh_precision */
   uint32_t path_slots;        /* 0 <=> automatic */
   uint32_t pending_entries;   /* per-path pending tally entries, 0 => 4 */
-  uint32_t graph_iterations;  /* 0: iterations driven from the host; n > 0:
-                                 n (rounded up to even) iterations captured
-                                 in a HIP graph and replayed until done */
+  uint32_t graph_iterations;  /* accepted, and changes nothing: one launch
+                                 takes every path a ray further, and one
+                                 runs the last few to their ends */
 };
 
 /* Several suns over the uploaded scene in one solve: sun j runs
@@ -496,10 +496,10 @@ SSOLH_API int ssolh_test_threefry
 SSOLH_API int ssolh_test_wave_sum
   (ssolh_context* ctx, uint32_t nwaves, const double* in, double* out);
 
-/* Traversal stack of the trace kernels: caps the entries each lane keeps in
- * LDS (16, 24 or 32; 0 restores the default, the smallest that holds the
- * scene's bound) for the solves that follow, so that the rest of the bound
- * goes to the device-memory overflow; *bound (if not NULL) = the uploaded
+/* Traversal stack of the renderer's trace kernel: caps the entries each lane
+ * keeps in LDS (16, 24 or 32; 0 restores the default, the smallest that holds
+ * the scene's bound) for the calls that follow, so that the rest of the bound
+ * goes to the device-memory overflow (the solver's kernels keep 20 or 32); *bound (if not NULL) = the uploaded
  * scene's bound (0 without a scene). The results do not depend on the cap. */
 SSOLH_API int ssolh_test_trace_stack(ssolh_context* ctx, uint32_t lds_cap, uint32_t* bound);
 
@@ -513,10 +513,9 @@ SSOLH_API int ssolh_test_slab_slack(ssolh_context* ctx, float scale);
 
 /* Log of per-primitive entries (finished paths append their entries; the
  * log is sorted by key and summed into the per-primitive tally after each
- * wavefront and whenever a host-driven iteration leaves it half full; a
- * full log sends further entries to per-lane atomics): caps it at `records`
- * entries for the solves that follow (0 restores the default, one per
- * realisation up to 2^27). *flushes and *overflowed (if not NULL) = the last
+ * wavefront and whenever a launch leaves it half full; a full log sends
+ * further entries to per-lane atomics): caps it at `records` entries for the
+ * solves that follow (0 restores the default, one per realisation up to 2^27). *flushes and *overflowed (if not NULL) = the last
  * solve's sorted reductions and the entries it sent to the atomics. The
  * results do not depend on the cap beyond the order of the additions. */
 SSOLH_API int ssolh_test_prim_log(ssolh_context* ctx, uint32_t records, uint32_t* flushes,

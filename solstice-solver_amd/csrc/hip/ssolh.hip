@@ -1,31 +1,27 @@
 // ssolh -- wavefront flux integrator on one MI355X (gfx950).
 //
 // Replaces the reference's OpenMP realisation loop (src/ssol_solver.c:
-// 1223-1248 running trace_radiative_path, :873-1127) by a wavefront of path
-// slots in HBM. Every per-path record (path state, next ray, last hit) is
-// indexed by its slot; the work list of an iteration is the list of slots
-// that have a ray to trace, kept in increasing slot order so that a wave
-// reads and writes contiguous runs of every record.
+// 1223-1248 running trace_radiative_path, :873-1127) by a wavefront: a lane
+// per realisation, and per launch one ray of every path in flight.
 //
-//   k_generate  fills the slots with new realisations (start point, sun
-//               direction, wavelength, weights) and writes their shadow rays;
-//   k_trace     one thread per listed slot: two-level BVH traversal in FP32
-//               boxes with the reference's any-hit filter inline
-//               (src/ssol_scene.c:438-536) and the FP64 quadric refinement
-//               (src/ssol_shape.c:1449-1494);
-//   k_shade     one thread per listed slot: the tail of the reference loop
-//               iteration that traced the ray (miss, segment extinction
-//               tallies, Russian roulette, point update) and the head of the
-//               next one (extinction, BSDF or virtual pass-through, receiver
-//               tallies); finished realisations flush their pending tallies
-//               with wave-aggregated FP64 atomics and, when the solve has
-//               more realisations than slots, the slot is refilled with its
-//               next realisation in place;
-//   k_scan_chunks / k_scan_top / k_scatter  order-preserving compaction of
-//               the slots that wrote a ray into the next work list (per-block
-//               counts, two-level scan of the counts, scatter).
+//   k_start     draws the realisations' start points, sun directions and
+//               wavelengths, traces their shadow rays and shades the start
+//               points;
+//   k_resume    takes the paths of a queue one ray further: two-level BVH
+//               traversal in FP32 boxes with the reference's any-hit filter
+//               inline (src/ssol_scene.c:438-536) and the FP64 quadric
+//               refinement (src/ssol_shape.c:1449-1494), then the tail of the
+//               reference loop iteration that traced the ray (miss, segment
+//               extinction, Russian roulette, point update) and the head of
+//               the next one (extinction, BSDF or virtual pass-through,
+//               receiver weights). Both leave the paths that go on in the
+//               next queue; finished realisations flush their tallies with
+//               wave-aggregated FP64 atomics;
+//   k_scan_chunks / k_scan_top / k_queue_list  list the queue's paths in the
+//               order they started in (waves' counts, two-level scan, list).
 //
-// The host loop runs trace / shade / scan / scatter until the list is empty.
+// The host launches k_resume until no path goes on, or few enough do for one
+// launch to run them through to their ends.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
@@ -49,9 +45,9 @@ using namespace ssolh;
 namespace {
 
 constexpr int BLOCK = 128;           // threads per block (2 waves)
-constexpr int WAVES = BLOCK / 64;
 constexpr int MAX_STACK = 32;        // traversal stack entries per thread in LDS, largest kernel
-constexpr int SCAN_THREADS = 1024;   // threads of a scan block
+constexpr uint32_t RUN_THROUGH = 1u << 18;  // a launch of at most so many paths runs them to their ends
+constexpr int START_STACK = 20, RESUME_STACK = 32;  // LDS stack entries per lane of the path kernels
 constexpr uint32_t SENTINEL = 0xFFFFFFFFu;
 constexpr uint32_t LEAF = 0x80000000u;
 constexpr uint32_t NONE = 0xFFFFFFFFu;
@@ -189,35 +185,15 @@ enum : uint32_t {
   PF_HIT_RECEIVER = 1u << 4    // the path reached a receiver (path tracking)
 };
 
-// The FP64 form keeps per slot only what a bounce changes plus a few
-// records written once per path; the position and direction of the point a
-// ray leaves are those of the ray record (its origin is the last real point,
-// also past a virtual one).
-struct PathState {
-  double2* cst;        // wavelength, cos factor (written once per path)
-  double4* pw;         // outgoing weights of the last real point (3); w: the
-                       // initial flux until the first shading, then the
-                       // incoming flux of the last virtual point crossed
-  double4* nrm;        // normal of the start point (written once per path)
-  double4* pend;       // pending absorbed_by_receivers, extinguished, other (first
-                       // written by the path's first shading, which starts from zeros)
-  uint4* st;           // path id lo/hi, rng block, flags
-  uint4* sm;           // (instance, shaded shape) index, prim, depth | side << 30,
-                       // in medium | out medium << 16
-  uint4* aux;          // sampled slot, job (written once per path), survivor
-                       // score, roulette interval (rewritten past depth 64)
-  uint32_t* pkey;      // [npend][slots]: receiver key (slot*2+side) or NONE
-  double* pval;        // [npend][10][slots]
-  uint32_t* qkey;      // [npend][slots]: per-primitive key or NONE
-  double* qval;        // [npend][10][slots]
-};
-
 struct Counters {
   unsigned long long failed;
   unsigned long long spills;
   unsigned long long segments;      // traced rays (added by k_scan_top, one thread)
   unsigned int aborted;
-  unsigned int pad;
+  unsigned int stop;                // aborted as the current wavefront began
+  unsigned int wavefronts;          // wavefronts begun
+  unsigned int iterations, gens;    // generations of rays: of the passes so far, of this one
+  unsigned int left;                // length of the list of paths that go on
 };
 
 // Tallies that every wave updates (global fields, counts) or that few keys
@@ -514,50 +490,6 @@ __global__ void k_iota32(uint32_t* a, uint32_t n) {
   if (i < n) a[i] = i;
 }
 
-// The logical blocks (of BLOCK list entries) of a looping, graph-captured
-// launch: the first 7/8 in static shares (block b to workgroup b mod grid),
-// the rest handed out in chunks from *fetch, which k_scan_top zeroes before
-// the next iteration. With static shares alone the kernel ends with its
-// slowest share; the handed-out tail lets the workgroups finish within about
-// one chunk of each other. A chunk is sized for about four tickets per
-// workgroup: one block per ticket made the atomics on *fetch (one address)
-// the bottleneck when the list stays full. Calls f(b) once for every block;
-// every thread of the workgroup must call it.
-template <typename F>
-__device__ __forceinline__ void for_each_block(uint32_t nb, unsigned* fetch, F&& f) {
-  __shared__ uint32_t s_b;
-  const uint32_t stat = nb - nb / 8;
-  const uint32_t chunk = max(1u, (nb - stat) / (gridDim.x * 4u));
-  uint32_t b = blockIdx.x, end = 0;  // uniform over the workgroup; [b, end): current chunk
-  for (;;) {
-    if (b >= stat && b >= end) {  // static share or chunk done: a new ticket
-      __syncthreads();  // every thread has read the previous ticket
-      if (threadIdx.x == 0) s_b = stat + atomicAdd(fetch, 1u) * chunk;
-      __syncthreads();
-      b = s_b;
-      if (b >= nb) break;
-      end = min(b + chunk, nb);
-    }
-    f(b);  // one call site: the block body is inlined once
-    b = b < stat ? b + gridDim.x : b + 1;
-  }
-}
-
-// Number of set predicates in the block, written by thread 0 to out[b]
-// (b: the logical block). Every thread of the block must call it.
-__device__ void block_count(bool pred, uint32_t* out, uint32_t b) {
-  __shared__ uint32_t wcount[WAVES];
-  const uint64_t m = __ballot(pred);
-  if (lane_id() == 0) wcount[threadIdx.x / 64] = (uint32_t)__popcll(m);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t s = 0;
-    for (int w = 0; w < WAVES; ++w) s += wcount[w];
-    out[b] = s;
-  }
-  __syncthreads();  // wcount is reused by the block's next logical block
-}
-
 // -------------------------------------------------------------------------
 // Traversal with the reference hit filter
 // -------------------------------------------------------------------------
@@ -647,6 +579,8 @@ __device__ __forceinline__ double ray_triangle(d3 o, const Shear& s, d3 v0, d3 v
   const double T = U * s.Sz * Az + V * s.Sz * Bz + W * s.Sz * Cz;
   return T / det;
 }
+
+struct ShapeQ;
 
 struct TraceState {
   double tbest;
@@ -902,49 +836,102 @@ struct TOvf {
   uint32_t stride, extra;
 };
 
-// STACK: LDS stack entries per lane (the smaller the stack, the more blocks
-// share a CU); the scene's bound beyond them goes to the overflow array. Four
-// waves per SIMD caps the kernel at 128 VGPRs; the few values that spill are
-// cold.
-// Entry q of the work list: traversal, filter, hit record
-template <int STACK>
-__device__ __forceinline__ void trace_ray(const DScene& S, const uint32_t* __restrict__ list,
-                                          uint32_t q, const RayRec* __restrict__ rays,
-                                          HitRec* __restrict__ hits, uint32_t* lds_stack,
-                                          const Node4* lds_top, const TOvf& ovf) {
-
-  const uint32_t slot = slot_of(list, q);
-  const RayRec r = rays[slot];
-  const d3 ow = mk(r.ox, r.oy, r.oz), dw = mk(r.dx, r.dy, r.dz);
-  const bool any_hit = (r.flags & RF_ANY_HIT) != 0;
+// What a traversal needs to know of one ray of the FP64 form: how it enters
+// an instance, tests a triangle against the filter and what it hit.
+struct Tracer64 {
+  using Ray = RayRec;
+  using Hit = HitRec;
+  const DScene& S;
+  const RayRec& r;
   TraceState ts;
-  ts.tbest = INFINITY;
-  ts.qdst = INFINITY;
-  ts.qiss = NONE;
-  ts.tri = 0;
-  ts.iss = NONE;
-  ts.prim = 0;
-  ts.punched = false;
+  d3 o, d;   // the ray in the frame of the instance being traversed
+  Shear sh;
 
-  TStack st{lds_stack + threadIdx.x, ovf.base ? ovf.base + q : nullptr, ovf.stride, ovf.extra, 0};
-  FRay fr = make_fray(ow, dw);
-  d3 o = ow, d = dw;        // current-level ray (double)
-  Shear sh = make_shear(dw);
-  bool in_blas = false;
-  uint32_t iss_first = 0;   // (instance, sshape) base of the BLAS being traversed
-  const float ftmin = r.tmin;
+  __device__ __forceinline__ Tracer64(const DScene& S_, const ShapeQ*, const RayRec& r_)
+      : S(S_), r(r_) {
+    ts.tbest = INFINITY;
+    ts.qdst = INFINITY;
+    ts.qiss = NONE;
+    ts.tri = 0;
+    ts.iss = NONE;
+    ts.prim = 0;
+    ts.punched = false;
+  }
+  __device__ __forceinline__ d3 ow() const { return mk(r.ox, r.oy, r.oz); }
+  __device__ __forceinline__ d3 dw() const { return mk(r.dx, r.dy, r.dz); }
+  __device__ __forceinline__ FRay world() const { return make_fray(ow(), dw()); }
   // A ray that leaves a point of a planar object can meet that object again
   // only at t ~ 0, which the filter rejects: its instance is not entered.
   // Nor is the instance of a one-shape object whose punched shape the ray
   // leaves when the filter could accept no candidate on it.
-  uint32_t skip_inst = NONE;
-  if (r.tmin == 0.f) {
+  __device__ __forceinline__ uint32_t skipped() const {
+    if (r.tmin != 0.f) return NONE;
     const IssInfo e = S.iss[r.iss_from];
     if ((e.obj_flags & SSOLH_OBJECT_PLANAR) ||
         ((e.obj_flags & OBJ_ONE_SHAPE) && e.shape_type != SSOLH_SHAPE_MESH &&
-         !punched_rehit_possible(S, r, ow, dw, r.iss_from, object_exit(S, e.inst, ow, dw))))
-      skip_inst = e.inst;
+         !punched_rehit_possible(S, r, ow(), dw(), r.iss_from, object_exit(S, e.inst, ow(), dw()))))
+      return e.inst;
+    return NONE;
   }
+  template <class InstPtr>
+  __device__ __forceinline__ FRay enter(InstPtr inst, uint32_t) {
+    const d3 T = mk(inst->transform[9], inst->transform[10], inst->transform[11]);
+    double m[9];
+    for (int k = 0; k < 9; ++k) m[k] = inst->inv_linear[k];
+    o = mul(m, ow() - T);
+    d = mul(m, dw());
+    sh = make_shear(d);
+    return make_fray(o, d);
+  }
+  // Triangle `tri`, item `index`: true if it is the new nearest hit; tmax:
+  // the box culling distance, the best hit so far widened by 2 ulp (FP32)
+  __device__ __forceinline__ bool hit(const ssolh_triangle& tri, uint32_t index,
+                                      uint32_t iss_first, float& tmax) {
+    const double t = ray_triangle(o, sh, ld3(tri.v0), ld3(tri.v1), ld3(tri.v2));
+    if (!(t >= r.tmin && t < ts.tbest)) return false;
+    d3 ng;
+    bool punched;
+    const uint32_t iss = iss_first + tri.sshape;
+    if (!filter(S, r, ow(), dw(), iss, tri, t, ts, ng, punched)) return false;
+    ts.tbest = t;
+    tmax = t < (double)FLT_MAX ? (float)t * 1.0000002f + 1e-30f : FLT_MAX;
+    ts.iss = iss;
+    ts.prim = tri.prim;
+    ts.tri = index;
+    ts.punched = punched;
+    return true;
+  }
+  __device__ __forceinline__ HitRec result() const {
+    HitRec h;
+    h.t = ts.tbest;
+    h.qdst = ts.qdst;
+    d3 n = mk(0, 0, 0);
+    if (ts.punched)
+      n = quadric_normal(S, ts.qiss, ow(), dw(), ts.qdst);
+    else if (ts.iss != NONE)
+      n = mesh_ng(S, S.iss[ts.iss].inst, S.tris[ts.tri]);
+    h.nx = n.x; h.ny = n.y; h.nz = n.z;
+    h.iss = ts.iss;
+    h.prim = ts.prim;
+    return h;
+  }
+};
+
+// One ray per lane, each on its own way through the tree. STACK: LDS stack
+// entries per lane (the smaller the stack, the more blocks share a CU); the
+// scene's bound beyond them goes to the overflow array, column q.
+template <class Tracer, int STACK>
+__device__ __forceinline__ typename Tracer::Hit
+trace_lane(const DScene& S, const ShapeQ* SQ, const typename Tracer::Ray& r, uint32_t q,
+           uint32_t* lds_stack, const Node4* lds_top, const TOvf& ovf) {
+  Tracer tr(S, SQ, r);
+  const bool any_hit = (r.flags & RF_ANY_HIT) != 0;
+  TStack st{lds_stack + threadIdx.x, ovf.base ? ovf.base + q : nullptr, ovf.stride, ovf.extra, 0};
+  FRay fr = tr.world();
+  bool in_blas = false;
+  uint32_t iss_first = 0;   // (instance, sshape) base of the BLAS being traversed
+  const float ftmin = r.tmin;
+  const uint32_t skip_inst = tr.skipped();
 
   // "while-while" traversal: the lanes of a wave first descend through inner
   // nodes together, then process their leaves together, which keeps the
@@ -952,7 +939,6 @@ __device__ __forceinline__ void trace_ray(const DScene& S, const uint32_t* __res
   // SENTINEL (all bits set) reads as a leaf reference and ends the descent.
   uint32_t ref = S.root_ref;
   bool alive = true;
-  // box culling distance: the best hit so far, widened by 2 ulp (FP32)
   float tmax = FLT_MAX;
   while (alive) {
     while (!(ref & LEAF)) {
@@ -969,9 +955,7 @@ __device__ __forceinline__ void trace_ray(const DScene& S, const uint32_t* __res
     if (ref == SENTINEL) {
       // back to the TLAS
       in_blas = false;
-      fr = make_fray(ow, dw);
-      o = ow;
-      d = dw;
+      fr = tr.world();
       alive = tpop<STACK>(st, ref);
       continue;
     }
@@ -983,76 +967,40 @@ __device__ __forceinline__ void trace_ray(const DScene& S, const uint32_t* __res
         alive = tpop<STACK>(st, ref);
         continue;
       }
-      const ssolh_instance& inst = S.insts[ii];
-      const d3 T = mk(inst.transform[9], inst.transform[10], inst.transform[11]);
-      o = mul(inst.inv_linear, ow - T);
-      d = mul(inst.inv_linear, dw);
-      fr = make_fray(o, d);
-      sh = make_shear(d);
-      iss_first = inst.isshape_first;
+      const ssolh_instance* inst = S.insts + ii;
+      fr = tr.enter(inst, ii);
+      iss_first = inst->isshape_first;
       in_blas = true;
       tpush<STACK>(st, SENTINEL);
-      ref = S.objects[inst.object].blas_root;
+      ref = S.objects[inst->object].blas_root;
       continue;
     }
     const uint32_t cnt = ((ref >> 28) & 7u) + 1u;
     bool done = false;
-    for (uint32_t k = 0; k < cnt; ++k) {
-      const ssolh_triangle tri = S.tris[first + k];
-      const double t = ray_triangle(o, sh, ld3(tri.v0), ld3(tri.v1), ld3(tri.v2));
-      if (!(t >= r.tmin && t < ts.tbest)) continue;
-      d3 ng;
-      bool punched;
-      const uint32_t iss = iss_first + tri.sshape;
-      if (!filter(S, r, ow, dw, iss, tri, t, ts, ng, punched)) continue;
-      ts.tbest = t;
-      tmax = t < (double)FLT_MAX ? (float)t * 1.0000002f + 1e-30f : FLT_MAX;
-      ts.iss = iss;
-      ts.prim = tri.prim;
-      ts.tri = first + k;
-      ts.punched = punched;
-      if (any_hit) { done = true; break; }
-    }
+    for (uint32_t k = 0; k < cnt && !done; ++k)
+      done = tr.hit(S.tris[first + k], first + k, iss_first, tmax) && any_hit;
     if (done) break;
     alive = tpop<STACK>(st, ref);
   }
-
-  HitRec h;
-  h.t = ts.tbest;
-  h.qdst = ts.qdst;
-  d3 n = mk(0, 0, 0);
-  if (ts.punched)
-    n = quadric_normal(S, ts.qiss, ow, dw, ts.qdst);
-  else if (ts.iss != NONE)
-    n = mesh_ng(S, S.iss[ts.iss].inst, S.tris[ts.tri]);
-  h.nx = n.x; h.ny = n.y; h.nz = n.z;
-  h.iss = ts.iss;
-  h.prim = ts.prim;
-  hits[slot] = h;
+  return tr.result();
 }
 
-// LOOP: graph-captured launch of a fixed grid, each block taking every
-// gridDim.x-th logical block of BLOCK list entries; else one logical block
-// per block
-template <int STACK, bool LOOP>
+// Rays of a work list from memory (the renderer's)
+template <int STACK>
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
 k_trace(DScene S, const uint32_t* __restrict__ list, const unsigned* __restrict__ count_ptr,
-        const RayRec* __restrict__ rays, HitRec* __restrict__ hits, unsigned* fetch, TOvf ovf) {
+        const RayRec* __restrict__ rays, HitRec* __restrict__ hits, TOvf ovf) {
   __shared__ uint32_t lds_stack[STACK * BLOCK];
   __shared__ Node4 lds_top[TOP_NODES];
   const uint32_t count = *count_ptr;
   if (blockIdx.x * BLOCK >= count) return;  // whole blocks only: the staging syncs
   for (uint32_t i = threadIdx.x; i < S.ntop; i += BLOCK) lds_top[i] = S.top[i];
   __syncthreads();
-  if (LOOP) {
-    for_each_block((count + BLOCK - 1) / BLOCK, fetch, [&](uint32_t b) {
-      const uint32_t q = b * BLOCK + threadIdx.x;
-      if (q < count) trace_ray<STACK>(S, list, q, rays, hits, lds_stack, lds_top, ovf);
-    });
-  } else {
-    const uint32_t q = blockIdx.x * BLOCK + threadIdx.x;
-    if (q < count) trace_ray<STACK>(S, list, q, rays, hits, lds_stack, lds_top, ovf);
-  }
+  const uint32_t q = blockIdx.x * BLOCK + threadIdx.x;
+  if (q >= count) return;
+  const uint32_t slot = slot_of(list, q);
+  const RayRec r = rays[slot];
+  hits[slot] = trace_lane<Tracer64, STACK>(S, nullptr, r, q, lds_stack, lds_top, ovf);
 }
 
 // -------------------------------------------------------------------------
@@ -1449,117 +1397,12 @@ k_lbvh_finish(uint32_t n, const uint32_t* __restrict__ skey, const uint32_t* __r
 }
 
 // -------------------------------------------------------------------------
-// Path generation (reference point_init, src/ssol_solver.c:207-358)
+// Paths
 // -------------------------------------------------------------------------
-struct Emit {
-  bool has;
-  RayRec r;
-};
-
 __device__ uint32_t start_medium(const DScene& S, const ssolh_material& m, uint32_t side) {
   if (m.type == SSOLH_MTL_DIELECTRIC || m.type == SSOLH_MTL_THIN_DIELECTRIC)
     return (uint32_t)(side == SSOL_FRONT_ ? m.medium_in : m.medium_out);
   return S.air;
-}
-
-// Sample triangle of a start point from the first uniform of its stream
-// (alias table over the sampling proxy, by area)
-__device__ __forceinline__ uint32_t alias_pick(const DScene& S, double u0) {
-  const double x = u0 * (double)S.nstris;
-  uint32_t i = (uint32_t)x;
-  if (i >= S.nstris) i = S.nstris - 1;
-  const ssolh_alias al = S.alias[i];
-  return (x - (double)i) < al.prob ? i : al.alias;
-}
-
-__device__ void generate(const DScene& S, const PathState& P, const SolveParams& prm,
-                         uint32_t slot, uint64_t path, Emit& e, int& samp_slot,
-                         const AdjParams& A, const TrackParams& K) {
-  PathRng rng;
-  rng.init(prm.key, prm.counter + path, 0);
-  // area-weighted primitive through the alias table, uniform point
-  const double u0 = rng.next(), u1 = rng.next(), u2 = rng.next();
-  const uint32_t idx = alias_pick(S, u0);
-  const ssolh_sample_tri st = S.stris[idx];
-  const ssolh_instance& inst = S.insts[st.instance];
-  const double sq = sqrt(u1);
-  const double b0 = 1 - sq, b1 = sq * (1 - u2), b2 = sq * u2;
-  const d3 v0 = ld3(st.v0), v1 = ld3(st.v1), v2 = ld3(st.v2);
-  const d3 T = mk(inst.transform[9], inst.transform[10], inst.transform[11]);
-  d3 pos = mul(inst.transform, v0 * b0 + v1 * b1 + v2 * b2) + T;
-  const d3 ns = normalize(tmul(inst.inv_linear, cross(v2 - v0, v1 - v0)));
-
-  const uint32_t job = job_of(prm, path);
-  const ssolh_sun& sun = job_sun(S, prm, job);
-  const d3 dir = sample_sun(sun, rng);
-  const double wl = sample_wavelength(S.spectra, sun.wl_spectrum, rng.next());
-
-  const uint32_t iss = inst.isshape_first + st.sshape;
-  const IssInfo is = S.iss[iss];
-  d3 N = ns;
-  const bool punched = is.shape_type == SSOLH_SHAPE_PUNCHED;
-  if (punched) {
-    // lift onto the quadric (src/ssol_shape.c:1408-1447)
-    const ssolh_shape& sh = S.shapes[is.shape];
-    const ssolh_inst_sshape& q = S.isshapes[iss];
-    d3 loc = mul(q.R_inv, pos - ld3(q.T));
-    loc.z = quadric_z(sh.quadric, sh.qparam, loc.x, loc.y);
-    N = normalize(tmul(q.R_inv, quadric_grad(sh.quadric, sh.qparam, loc)));
-    pos = mul(q.R, loc) + ld3(q.T);
-  }
-  uint32_t side = SSOL_FRONT_;
-  if (dot(N, dir) >= 0) { side = SSOL_BACK_; N = -N; }
-
-  const d3 sun0 = ld3(sun.dir);
-  const double surface_sun_cos = dot(N, dir);
-  const double surface_sun0_cos = fabs(dot(sun0, N));
-  const double sun0_sun_cos = dot(sun0, dir);
-  const double proxy_cos = punched ? fabs(dot(ns, N)) : 1.0;
-  const double w0 = sun.dni * S.S_proxy * fabs(surface_sun_cos / (proxy_cos * sun0_sun_cos));
-  const double cosf = S.S_proxy / S.S * surface_sun0_cos / proxy_cos;
-
-  const ssolh_material& m = S.mtls[side == SSOL_FRONT_ ? is.mtl_front : is.mtl_back];
-  const uint32_t med = start_medium(S, m, side);
-
-  if (K.vtx) {
-    // sun point and start point (src/ssol_solver.c:909-921)
-    K.seq[slot] = 0;
-    if (K.sun_len > 0) track_vertex(K, slot, path, pos - dir * K.sun_len, sun.dni);
-    track_vertex(K, slot, path, pos, w0);
-  }
-
-  if (A.grad) {
-    // w0 is proportional to |N.w|: d log w0 / d angle = ((a x N).w) / (N.w)
-    const int32_t pp = A.inst_param[st.instance];
-    double4 sc = make_double4(0, 0, 0, 0);
-    if (pp >= 0) {
-      const d3 a1 = ld3(A.axes + 6 * pp), a2 = ld3(A.axes + 6 * pp + 3);
-      sc.x = dot(cross(a1, N), dir) / surface_sun_cos;
-      sc.y = dot(cross(a2, N), dir) / surface_sun_cos;
-    }
-    A.s[slot] = sc;
-    A.p[slot] = pp >= 0 ? (uint32_t)pp : NONE;
-  }
-
-  if (K.vtx) K.pos[slot] = make_double4(pos.x, pos.y, pos.z, 0);
-  P.cst[slot] = make_double2(wl, cosf);
-  P.pw[slot] = make_double4(w0, w0, w0, w0);
-  P.nrm[slot] = make_double4(N.x, N.y, N.z, 0);
-  P.st[slot] = make_uint4((uint32_t)path, (uint32_t)(path >> 32), rng.block, PF_ACTIVE);
-  P.sm[slot] = make_uint4(iss, st.prim, 0u | (side << 30), med | (med << 16));
-  P.aux[slot] = make_uint4((uint32_t)inst.sampled, job, 0, 64u);
-  // the slot's pending keys are all NONE already (cleared with the state,
-  // and by the flush of the slot's previous realisation)
-  samp_slot = inst.sampled;
-
-  // shadow ray toward the sun (src/ssol_solver.c:325-352)
-  e.has = true;
-  e.r.ox = pos.x; e.r.oy = pos.y; e.r.oz = pos.z;
-  e.r.dx = -dir.x; e.r.dy = -dir.y; e.r.dz = -dir.z;
-  e.r.tmin = 0;
-  e.r.iss_from = iss;
-  e.r.prim_from = st.prim;
-  e.r.flags = (side << RF_SIDE_SHIFT) | RF_DISCARD_VIRTUAL | RF_REVERSED | RF_ANY_HIT;
 }
 
 __device__ void flush_sampled_count(bool has, int samp_slot, const Tallies& T) {
@@ -1575,666 +1418,12 @@ __device__ void flush_sampled_count(bool has, int samp_slot, const Tallies& T) {
   if (has && !match) atomicAdd(base + key, 1ull);
 }
 
-// First realisations of a wavefront: slot s holds realisation first +
-// order[s] (first + s when order is null), s < count, order a permutation
-// of [0, count). With refill, slot s then runs that realisation + k * slots,
-// k = 1, 2, ... while below N. Four waves per SIMD (at most 128 VGPRs, 44
-// bytes per lane spilled) run it faster than three without spills (10k
-// field: 8.20 -> 7.59 ms per 1e8 realisations; five: 9.65 ms).
-template <bool ADJ>
-__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
-k_generate(DScene S, PathState P, SolveParams prm, Tallies T, RayRec* __restrict__ rays,
-           uint64_t first, uint32_t count, AdjParams A_, TrackParams K,
-           const uint32_t* __restrict__ order) {
-  const AdjParams A = ADJ ? A_ : AdjParams{};
-  const uint32_t slot = blockIdx.x * BLOCK + threadIdx.x;
-  const bool live = slot < count;
-  Emit e;
-  e.has = false;
-  int samp_slot = 0;
-  if (live) generate(S, P, prm, slot, first + (order ? order[slot] : slot), e, samp_slot, A, K);
-  flush_sampled_count(live, samp_slot, T);
-  if (e.has) rays[slot] = e.r;
-}
-
-// -------------------------------------------------------------------------
-// Shading (reference trace_radiative_path loop body, src/ssol_solver.c:939-1086)
-// -------------------------------------------------------------------------
 enum { FIN_NONE = 0, FIN_DONE = 1, FIN_KILLED = 2, FIN_FAILED = 3 };
 
-struct Finish {
-  int kind;
-  double g[6];      // cos, absorbed_by_receivers, shadowed, missing, extinct, other
-  double factor;    // survivor factor applied to pending entries
-  int samp_slot;
-  uint32_t job;     // sun of the realisation
-};
-
-// Add the 10 receiver weights of a hit to the per-path pending entries;
-// false when every entry holds another key.
-__device__ bool pend_add(uint32_t* keys, double* vals, size_t stride, uint32_t npend,
-                         uint32_t key, const double* w) {
-  int slot_k = -1, free_k = -1;
-  uint32_t kk[MAX_PEND];
-#pragma unroll
-  for (int k = 0; k < MAX_PEND; ++k) kk[k] = (uint32_t)k < npend ? keys[k * stride] : 0u;
-#pragma unroll
-  for (int k = MAX_PEND - 1; k >= 0; --k) {
-    if ((uint32_t)k >= npend) continue;
-    if (kk[k] == key) slot_k = k;
-    if (kk[k] == NONE) free_k = k;
-  }
-  if (slot_k < 0 && free_k >= 0) {
-    slot_k = free_k;
-    keys[slot_k * stride] = key;
-    for (int f = 0; f < 10; ++f) vals[((size_t)slot_k * 10 + f) * stride] = 0;
-  }
-  if (slot_k < 0) return false;
-  for (int f = 0; f < 10; ++f) vals[((size_t)slot_k * 10 + f) * stride] += w[f];
-  return true;
-}
-
-// Weights that found no pending entry are flushed as a term of their own
-__device__ void spill(double* base, uint64_t key, const double* w, unsigned long long* spills) {
-  atomicAdd(spills, 1ull);
-  for (int f = 0; f < 10; ++f) {
-    atomic_add(base + key * 20 + 2 * f, w[f]);
-    atomic_add(base + key * 20 + 2 * f + 1, w[f] * w[f]);
-  }
-}
-
-// Logical block b (list entries b*BLOCK ...) of k_shade; ADJ: the adjoint
-// solve's variant, the plain one carries no score code; REFILL: slots take
-// further realisations (fewer slots than realisations), without it no
-// generation code.
-template <bool ADJ, bool REFILL>
-__device__ __forceinline__ void shade_block(
-    uint32_t b, const DScene& S, const PathState& P, const SolveParams& prm, const Tallies& T,
-    const uint32_t* __restrict__ list, uint32_t count, RayRec* __restrict__ rays,
-    const HitRec* __restrict__ hits, uint8_t* __restrict__ emitted,
-    uint32_t* __restrict__ block_emits, Counters* C, const AdjParams& A_, const TrackParams& K) {
-  const AdjParams A = ADJ ? A_ : AdjParams{};
-  const uint32_t q = b * BLOCK + threadIdx.x;
-  const bool live = q < count;
-  const size_t stride = prm.slots;
-
-  Emit e;
-  e.has = false;
-  Finish fin;
-  fin.kind = FIN_NONE;
-  fin.factor = 1;
-  fin.samp_slot = 0;
-  fin.job = 0;
-  for (int i = 0; i < 6; ++i) fin.g[i] = 0;
-  const uint32_t slot = live ? slot_of(list, q) : 0;
-  // receiver weights of a hit that ends the path: flushed from registers
-  // below rather than stored as pending entries and read back (dkey, dpkey:
-  // receiver and per-primitive keys, NONE: no such hit)
-  uint32_t dkey = NONE, dpkey = NONE;
-  double din[4] = {0, 0, 0, 0};  // in0, in1, in2, kabs of that hit
-
-  uint64_t path = 0;
-  if (live) {
-    const HitRec h = hits[slot];
-    const uint4 st = P.st[slot];
-    const uint4 sm = P.sm[slot];
-    const double2 cw = P.cst[slot];
-    // outgoing weights of the last real point (3); w: the initial flux
-    // before the first shading, then the incoming flux of the last virtual
-    // point the path crossed
-    double4 pv = P.pw[slot];
-    double4 pd = (st.w & PF_STAGE_BOUNCE) ? P.pend[slot] : make_double4(0, 0, 0, 0);
-    // the ray of the emitting point: its origin (the last real point, also
-    // past a virtual point, whose ray keeps that origin) and direction
-    const RayRec& rr = rays[slot];
-    const d3 rorg0 = mk(rr.ox, rr.oy, rr.oz), rdir0 = mk(rr.dx, rr.dy, rr.dz);
-    path = (uint64_t)st.x | ((uint64_t)st.y << 32);
-    PathRng rng;
-    rng.init(prm.key, prm.counter + path, st.z);
-    const uint32_t flags0 = st.w;
-    uint32_t flags = flags0;
-    uint32_t iss = sm.x, prim = sm.y;
-    uint32_t depth = sm.z & 0x3FFFFFFFu, side = sm.z >> 30;
-    uint32_t in_med = sm.w & 0xFFFFu, out_med = sm.w >> 16;
-    // sampled slot, job, survivor score and roulette interval: read at the
-    // end of the path and past the first roulette depth only
-    uint4 aux = make_uint4(0, 0, 0, 64);
-    bool have_aux = false;
-    auto load_aux = [&]() {
-      if (!have_aux) { aux = P.aux[slot]; have_aux = true; }
-    };
-    const double wl = cw.x;
-    d3 pos = rorg0;
-    d3 dir = (flags & PF_STAGE_BOUNCE) ? rdir0 : -rdir0;  // the shadow ray points at the sun
-    d3 N = mk(0, 0, 0);
-    if (!(flags & PF_STAGE_BOUNCE)) {
-      // normal of the start point (later points take theirs from the hit)
-      const double4 nt = P.nrm[slot];
-      N = mk(nt.x, nt.y, nt.z);
-    }
-    double hit_t = 0;
-    d3 rorg = pos, rdir = dir;  // origin/direction of the ray of the point
-    bool head = false;
-
-    if (!(flags & PF_STAGE_BOUNCE)) {
-      // result of the shadow ray
-      if (h.iss != NONE) {
-        fin.kind = FIN_DONE;
-        fin.g[2] = pv.w;      // shadowed = initial flux
-      } else {
-        head = true;
-        hit_t = 0;
-      }
-    } else {
-      // tail of the iteration that traced this ray
-      const bool found = h.iss != NONE;
-      const bool hit_virtual = (flags & PF_HIT_VIRTUAL) != 0;
-      const bool in_atm = (flags & PF_IN_ATM) != 0;
-      // flux that left the emitting point
-      const double left = hit_virtual ? pv.w : pv.x;
-      if (!found) {
-        // escape point (src/ssol_solver.c:1012-1019)
-        if (K.vtx && K.inf_len > 0) {
-          const double4 kp = K.pos[slot];
-          track_vertex(K, slot, path, mk(kp.x, kp.y, kp.z) + dir * K.inf_len, left);
-        }
-        if (out_med != S.air) {
-          fin.kind = FIN_FAILED;  // ray lost outside air
-        } else {
-          // past a virtual point the segment from the last real point
-          // ends at the virtual one (a real point's segment was counted
-          // at that point)
-          if (hit_virtual) {
-            const double absorbed = pv.x - pv.w;
-            if (in_atm) pd.y += absorbed; else pd.z += absorbed;
-          }
-          fin.kind = FIN_DONE;
-          fin.g[3] = left;  // missing
-        }
-      }
-      if (fin.kind == FIN_NONE) {
-        depth += hit_virtual ? 0u : 1u;
-        if (depth > 64) {
-          load_aux();
-          const uint32_t rinterval = aux.w;
-          if (depth > rinterval && depth % rinterval == 1) {
-            if (rng.next() > 0.5) {
-              aux.z += 1;
-              aux.w = 16;
-              P.aux[slot] = aux;
-            } else {
-              fin.kind = FIN_KILLED;
-            }
-          }
-        }
-      }
-      if (fin.kind == FIN_NONE) {
-        // point_update_from_hit (src/ssol_solver.c:360-411)
-        rorg = rorg0;
-        rdir = dir;
-        iss = h.iss;
-        prim = h.prim;
-        N = normalize(mk(h.nx, h.ny, h.nz));
-        if (S.iss[iss].shape_type == SSOLH_SHAPE_MESH) pos = rorg + rdir * h.t;
-        else pos = rorg + dir * h.qdst;
-        if (dot(dir, N) < 0) side = SSOL_FRONT_;
-        else { side = SSOL_BACK_; N = -N; }
-        in_med = out_med;
-        hit_t = h.t;
-        head = true;
-        if (K.vtx) track_vertex(K, slot, path, pos, left);  // src/ssol_solver.c:1080-1083
-      }
-    }
-
-    if (head) {
-      if (!(flags & PF_STAGE_BOUNCE)) { rorg = pos; rdir = dir; }
-      const IssInfo is = S.iss[iss];
-      const ssolh_material& m = S.mtls[side == SSOL_FRONT_ ? is.mtl_front : is.mtl_back];
-      const bool in_atm = in_med == S.air;
-      const bool receiver = (is.receiver_mask & side) != 0;
-      const bool virt = m.type == SSOLH_MTL_VIRTUAL;
-      if (receiver) flags |= PF_HIT_RECEIVER;
-      double trans = 1;
-      if (hit_t > 0) {
-        const double k = data_value(S.spectra, S.media[in_med].extinction, wl);
-        if (k > 0) trans = exp(-k * hit_t);
-      }
-      const double in0 = pv.x * trans;
-      const double in1 = in_atm ? pv.y : pv.y * trans;
-      const double in2 = !in_atm ? pv.z : pv.z * trans;
-      double out0, out1, out2, kabs;
-      uint32_t next_med = in_med;
-      if (virt) {
-        out0 = in0; out1 = in1; out2 = in2; kabs = 0;
-      } else {
-        double eta_out = 1, eta_in = 1, slab_eta = 1, slab_abs = 0;
-        if (m.type == SSOLH_MTL_DIELECTRIC) {
-          if ((uint32_t)m.medium_out != in_med) fin.kind = FIN_FAILED;
-          eta_out = data_value(S.spectra, S.media[m.medium_out].refractive_index, wl);
-          eta_in = data_value(S.spectra, S.media[m.medium_in].refractive_index, wl);
-        } else if (m.type == SSOLH_MTL_THIN_DIELECTRIC) {
-          eta_out = data_value(S.spectra, S.media[m.medium_out].refractive_index, wl);
-          slab_eta = data_value(S.spectra, m.slab_eta, wl);
-          slab_abs = data_value(S.spectra, m.slab_absorption, wl);
-        }
-        double w = 0;
-        int lobe = LOBE_NONE;
-        const d3 wi = -dir;
-        if (fin.kind == FIN_NONE && dot(wi, N) > 0) {
-          d3 wo, hm = N;
-          w = bsdf_sample(m, eta_out, eta_in, slab_eta, slab_abs, wi, N, rng, wo, lobe, &hm);
-          const double c = dot(N, wo);
-          if ((c > 0 && lobe == LOBE_TRANSMIT) || (c < 0 && lobe == LOBE_REFLECT)) w = 0;
-          dir = wo;
-          if (A.grad && !(flags & PF_STAGE_BOUNCE) && w > 0 && m.type == SSOLH_MTL_MIRROR &&
-              m.roughness > 0 && m.distribution == 0) {
-            // first reflection of a path that starts on a parameterised
-            // heliostat: score of the Beckmann microfacet density
-            // p(h) = exp(-tan^2/m^2) / (pi m^2 cos^3) under a rotation of
-            // the macro normal N about axis a (dN = a x N) and under m:
-            //   dlog p/d angle = (2 sec^2/m^2 - 3) sec (h . (a x N))
-            //   dlog p/dm      = 2 tan^2/m^3 - 2/m,  m = sqrt(2) slope error
-            const uint32_t pp = A.p[slot];
-            if (pp != NONE) {
-              const double ct = fmin(dot(hm, N), 1.0);
-              const double sec = 1.0 / ct, t2 = sec * sec - 1.0;
-              const double mr = m.roughness;
-              const double k = (2.0 * sec * sec / (mr * mr) - 3.0) * sec;
-              const d3 a1 = ld3(A.axes + 6 * pp), a2 = ld3(A.axes + 6 * pp + 3);
-              double4 sc = A.s[slot];
-              sc.x += k * dot(hm, cross(a1, N));
-              sc.y += k * dot(hm, cross(a2, N));
-              sc.z += 1.4142135623730951 * (2.0 * t2 / (mr * mr * mr) - 2.0 / mr);
-              A.s[slot] = sc;
-            }
-          }
-        }
-        kabs = 1 - w;
-        out0 = in0 * w;
-        out1 = in1 * w;
-        out2 = receiver ? in2 * w : in2;
-        if (lobe == LOBE_TRANSMIT && m.type == SSOLH_MTL_DIELECTRIC)
-          next_med = (uint32_t)(m.medium_out == (int32_t)in_med ? m.medium_in : m.medium_out);
-      }
-      if (fin.kind == FIN_NONE) {
-        if (receiver) {
-          pd.x += in0 - out0;
-          double w10[10];
-          w10[0] = in0; w10[1] = in1; w10[2] = in2;
-          w10[3] = in2 - in0; w10[4] = in1 - in0;
-          w10[5] = in0 * kabs; w10[6] = in1 * kabs; w10[7] = in2 * kabs;
-          w10[8] = (in2 - in0) * kabs; w10[9] = (in1 - in0) * kabs;
-          const uint32_t rkey = (uint32_t)is.receiver * 2u + (side == SSOL_FRONT_ ? 0u : 1u);
-          // the path ends at this point (weight zero below): its weights
-          // join the end-of-path flush directly
-          const bool direct = out0 == 0;
-          if (direct) {
-            dkey = rkey;
-            din[0] = in0; din[1] = in1; din[2] = in2; din[3] = kabs;
-          } else if (!pend_add(P.pkey + slot, P.pval + slot, stride, prm.npend, rkey, w10)) {
-            load_aux();
-            spill(T.rcv + (size_t)(blockIdx.x & T.mask_r) * T.nrcv * 40u, rkey, w10, &C->spills);
-            spill(T.sxr + (size_t)(blockIdx.x & T.mask_x) * T.nsamp * T.nrcv * 40u, (uint64_t)aux.x * S.nrcv * 2u + rkey, w10, &C->spills);
-          }
-          if (is.prim_tally >= 0) {
-            const uint32_t pkey = (uint32_t)(((uint64_t)is.prim_tally + prim) * 2u +
-                                             (side == SSOL_FRONT_ ? 0u : 1u));
-            if (direct)
-              dpkey = pkey;
-            else if (!pend_add(P.qkey + slot, P.qval + slot, stride, prm.npend, pkey, w10))
-              spill(T.prim + (size_t)(blockIdx.x & T.mask_p) * T.nprim * 40u, pkey, w10, &C->spills);
-            if (A.grad && A.p[slot] != NONE) A.s[slot].w += A.gmap[pkey] * w10[5];
-          }
-          if (A.grad && A.p[slot] != NONE) A.s[slot].w += A.d_total * (in0 - out0);
-        } else {
-          pd.z += in0 * kabs;
-        }
-        // extinction of the segment that reached this point, counted here at
-        // a real point (past virtual points the segment runs from the last
-        // real point); a virtual point counts it only if the path ends
-        if (!virt || out0 == 0) {
-          const double absorbed = pv.x - in0;
-          if (in_atm) pd.y += absorbed; else pd.z += absorbed;
-        }
-        if (out0 == 0) {
-          // weight is zero: the segment ends here
-          fin.kind = FIN_DONE;
-          fin.g[3] = 0;
-        } else {
-          e.has = true;
-          if (virt) {
-            e.r.ox = rorg.x; e.r.oy = rorg.y; e.r.oz = rorg.z;
-            e.r.dx = rdir.x; e.r.dy = rdir.y; e.r.dz = rdir.z;
-            e.r.tmin = nextafterf((float)hit_t, FLT_MAX);
-            pv.w = in0;
-          } else {
-            e.r.ox = pos.x; e.r.oy = pos.y; e.r.oz = pos.z;
-            e.r.dx = dir.x; e.r.dy = dir.y; e.r.dz = dir.z;
-            e.r.tmin = 0;
-            pv = make_double4(out0, out1, out2, pv.w);
-          }
-          e.r.iss_from = iss;
-          e.r.prim_from = prim;
-          e.r.flags = side << RF_SIDE_SHIFT;
-          flags = (flags & PF_HIT_RECEIVER) | PF_ACTIVE | PF_STAGE_BOUNCE |
-                  (virt ? PF_HIT_VIRTUAL : 0u) | (in_atm ? PF_IN_ATM : 0u);
-          out_med = next_med;
-        }
-      }
-    }
-
-    if (fin.kind != FIN_NONE) {
-      load_aux();
-      fin.samp_slot = (int)aux.x;
-      fin.job = aux.y;
-    }
-    if (K.vtx && fin.kind != FIN_NONE) {
-      // path type (src/ssol_solver.c:931, 1092-1094, 1111-1125)
-      uint8_t ty;
-      if (fin.kind == FIN_KILLED) ty = SSOLH_PATH_DROPPED;
-      else if (fin.kind == FIN_FAILED) ty = SSOLH_PATH_ERROR;
-      else if (!(flags0 & PF_STAGE_BOUNCE) && h.iss != NONE) ty = SSOLH_PATH_SHADOW;
-      else ty = (flags & PF_HIT_RECEIVER) ? SSOLH_PATH_SUCCESS : SSOLH_PATH_MISSING;
-      K.type[path] = ty;
-    }
-    if (fin.kind == FIN_DONE) {
-      fin.g[0] = cw.y;  // cos factor
-      fin.g[1] = pd.x;
-      fin.g[4] = pd.y;
-      fin.g[5] = pd.z;
-      fin.factor = (double)(1u << aux.z);
-      for (int i = 0; i < 6; ++i) fin.g[i] *= fin.factor;
-    }
-    if (fin.kind == FIN_NONE) {
-      P.pw[slot] = pv;
-      P.pend[slot] = pd;
-      P.st[slot] = make_uint4(st.x, st.y, rng.block, flags);
-      P.sm[slot] = make_uint4(iss, prim, depth | (side << 30), in_med | (out_med << 16));
-      if (K.vtx) K.pos[slot] = make_double4(pos.x, pos.y, pos.z, 0);
-    }
-  }
-
-  // --- convergent flush of finished realisations -------------------------
-  const bool done = fin.kind == FIN_DONE;
-  double* rcv_base = T.rcv + (size_t)(blockIdx.x & T.mask_r) * T.nrcv * 40u;
-  {
-    // global fields and the realisation count of the path's job (sun)
-    const bool counted = done || fin.kind == FIN_KILLED;
-    double g2[13];
-    for (int i = 0; i < 6; ++i) {
-      g2[2 * i] = done ? fin.g[i] : 0.0;
-      g2[2 * i + 1] = done ? fin.g[i] * fin.g[i] : 0.0;
-    }
-    g2[12] = 1.0;
-    keyed_add<13, 16>(counted, counted ? fin.job : 0, g2,
-                      T.global + (size_t)(blockIdx.x & T.mask_g) * T.njobs * 16u);
-    double s4[4] = {fin.g[0], fin.g[0] * fin.g[0], fin.g[2], fin.g[2] * fin.g[2]};
-    keyed_add<4>(done, (uint64_t)fin.samp_slot, s4,
-                 T.samp + (size_t)(blockIdx.x & T.mask_s) * T.nsamp * 4u);
-    const unsigned long long nf = wave_count_add(fin.kind == FIN_FAILED, &C->failed);
-    if (fin.kind == FIN_FAILED && nf + 1 >= prm.max_failed) atomicExch(&C->aborted, 1u);
-  }
-  // pending entries fill from entry 0 up (pend_add takes the lowest free
-  // one), so a path's keys end at its first empty entry and the wave stops
-  // at the first entry none of its finished paths uses
-  // The weights of the hit that ended the path (a direct entry) join the
-  // pending entry of the same key if the path holds one, before squaring;
-  // else they take the path's first empty entry position, one past the
-  // pending entries at most.
-  bool more = live && fin.kind != FIN_NONE;
-  bool dpend = done && dkey != NONE;
-  double dw[10];
-  dw[0] = din[0]; dw[1] = din[1]; dw[2] = din[2];
-  dw[3] = din[2] - din[0]; dw[4] = din[1] - din[0];
-  dw[5] = din[0] * din[3]; dw[6] = din[1] * din[3]; dw[7] = din[2] * din[3];
-  dw[8] = (din[2] - din[0]) * din[3]; dw[9] = (din[1] - din[0]) * din[3];
-  for (uint32_t k = 0; k <= prm.npend; ++k) {
-    uint32_t key = NONE;
-    double a10[10];
-    if (more && k < prm.npend) {
-      key = P.pkey[k * stride + slot];
-      if (key != NONE) {
-        const bool merge = dpend && key == dkey;
-        for (int f = 0; f < 10; ++f)
-          a10[f] = P.pval[((size_t)k * 10 + f) * stride + slot] + (merge ? dw[f] : 0.0);
-        if (merge) dpend = false;
-        P.pkey[k * stride + slot] = NONE;
-      }
-    }
-    if (key == NONE) {
-      more = false;
-      if (dpend) {
-        key = dkey;
-        for (int f = 0; f < 10; ++f) a10[f] = dw[f];
-        dpend = false;
-      }
-    }
-    if (!__ballot(key != NONE)) break;
-    const bool has = done && key != NONE;
-    double v[20];
-    for (int f = 0; f < 10; ++f) {
-      const double x = has ? a10[f] * fin.factor : 0.0;
-      v[2 * f] = x;
-      v[2 * f + 1] = x * x;
-    }
-    keyed_add<20>(has, has ? key : 0, v, rcv_base);
-    const uint64_t xkey = has ? (uint64_t)fin.samp_slot * (uint64_t)S.nrcv * 2u + key : 0;
-    keyed_add<20>(has, xkey, v, T.sxr + (size_t)(blockIdx.x & T.mask_x) * T.nsamp * T.nrcv * 40u);
-  }
-  more = live && fin.kind != FIN_NONE;  // per-primitive entries, the same way
-  dpend = done && dpkey != NONE;
-  for (uint32_t k = 0; k <= prm.npend; ++k) {
-    uint32_t key = NONE;
-    double a10[10];
-    if (more && k < prm.npend) {
-      key = P.qkey[k * stride + slot];
-      if (key != NONE) {
-        const bool merge = dpend && key == dpkey;
-        for (int f = 0; f < 10; ++f)
-          a10[f] = P.qval[((size_t)k * 10 + f) * stride + slot] + (merge ? dw[f] : 0.0);
-        if (merge) dpend = false;
-        P.qkey[k * stride + slot] = NONE;
-      }
-    }
-    if (key == NONE) {
-      more = false;
-      if (dpend) {
-        key = dpkey;
-        for (int f = 0; f < 10; ++f) a10[f] = dw[f];
-        dpend = false;
-      }
-    }
-    if (!__ballot(key != NONE)) break;
-    prim_add(T, done && key != NONE, key, a10, fin.factor);
-  }
-
-  // --- adjoint: the finished path's weighted contribution times its scores,
-  // wave-reduced (in start-instance order a wave's paths share a heliostat)
-  if (A.grad) {
-    const uint32_t pp = done ? A.p[slot] : NONE;
-    const bool has = pp != NONE;
-    double v[3] = {0.0, 0.0, 0.0};
-    if (has) {
-      const double4 sc = A.s[slot];
-      const double q = sc.w * fin.factor;
-      v[0] = q * sc.x;
-      v[1] = q * sc.y;
-      v[2] = q * sc.z;
-    }
-    keyed_add<3>(has, has ? pp : 0u, v, A.grad);
-  }
-
-  // --- refill finished slots with their next realisation -------------------
-  const bool want = live && fin.kind != FIN_NONE && !C->aborted;
-  const uint64_t id = want ? path + prm.slots : 0;
-  int samp_slot = 0;
-  bool gen = false;
-  if (REFILL && want && id < prm.N) {
-    generate(S, P, prm, slot, id, e, samp_slot, A, K);
-    gen = true;
-  }
-  flush_sampled_count(gen, samp_slot, T);
-
-  // --- the slot's next ray and its place in the next work list -----------
-  if (e.has) rays[slot] = e.r;
-  if (live) emitted[slot] = e.has ? 1 : 0;
-  block_count(e.has, block_emits, b);
-}
-
-// The arguments of a shade kernel in one struct: the struct is the kernel's
-// argument segment (offset 0), which a looping launch reads again for each
-// logical block (kernel_args)
-struct ShadeArgs {
-  DScene S;
-  PathState P;
-  SolveParams prm;
-  Tallies T;
-  const uint32_t* list;
-  const unsigned* count;
-  RayRec* rays;
-  const HitRec* hits;
-  uint8_t* emitted;
-  uint32_t* block_emits;
-  Counters* C;
-  AdjParams A;
-  TrackParams K;
-  unsigned* fetch;  // tail-block counter of a looping launch (for_each_block)
-};
-
-// The kernel's argument segment as an Args, behind a pointer the compiler
-// cannot see through. A looping kernel takes it anew for each logical
-// block, so the scalar loads of the arguments stay next to their uses: hoisted
-// out of the loop, the dozens of argument words would be held in scalar
-// registers across it and spill (through vector registers into scratch).
-template <typename Args>
-__device__ __forceinline__ const Args& kernel_args() {
-  auto p = (const __attribute__((address_space(4))) Args*)__builtin_amdgcn_kernarg_segment_ptr();
-  asm volatile("" : "+s"(p));
-  return *(const Args*)p;
-}
-
-template <bool ADJ, bool REFILL, bool LOOP>
-__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3)))
-k_shade(ShadeArgs a) {
-  const uint32_t count = *a.count;
-  // whole logical blocks only: block_count syncs (LOOP: as in k_trace)
-  if (LOOP) {
-    for_each_block((count + BLOCK - 1) / BLOCK, a.fetch, [&](uint32_t b) {
-      const ShadeArgs& f = kernel_args<ShadeArgs>();
-      shade_block<ADJ, REFILL>(b, f.S, f.P, f.prm, f.T, f.list, count, f.rays, f.hits, f.emitted,
-                               f.block_emits, f.C, f.A, f.K);
-    });
-  } else if (blockIdx.x * BLOCK < count) {
-    shade_block<ADJ, REFILL>(blockIdx.x, a.S, a.P, a.prm, a.T, a.list, count, a.rays, a.hits,
-                             a.emitted, a.block_emits, a.C, a.A, a.K);
-  }
-}
-
-// -------------------------------------------------------------------------
-// Order-preserving compaction of the work list
-// -------------------------------------------------------------------------
-// Exclusive scan of the per-block emit counts of k_shade in two levels:
-// k_scan_chunks scans each chunk of SCAN_CHUNK counts (offsets within the
-// chunk) and records the chunk's total; k_scan_top scans the chunk totals in
-// place into chunk offsets and writes the grand total, the next list's
-// length. Entry b of the scan is offsets[b] + chunk[b / SCAN_CHUNK].
-constexpr int SCAN_PER = 4;
-constexpr int SCAN_CHUNK = SCAN_THREADS * SCAN_PER;
-static_assert((1u << 28) / BLOCK / SCAN_CHUNK <= SCAN_THREADS, "one k_scan_top block scans every chunk");
-
-__device__ void block_inclusive_scan(uint32_t* part) {
-  const uint32_t tid = threadIdx.x;
-  for (uint32_t off = 1; off < SCAN_THREADS; off <<= 1) {
-    const uint32_t v = tid >= off ? part[tid - off] : 0u;
-    __syncthreads();
-    part[tid] += v;
-    __syncthreads();
-  }
-}
-
-__global__ void __launch_bounds__(SCAN_THREADS)
-k_scan_chunks(const uint32_t* __restrict__ counts, const unsigned* __restrict__ count_ptr,
-              uint32_t* __restrict__ offsets, uint32_t* __restrict__ chunk) {
-  __shared__ uint32_t part[SCAN_THREADS];
-  const uint32_t nblocks = (*count_ptr + BLOCK - 1) / BLOCK;
-  const uint32_t base = blockIdx.x * SCAN_CHUNK;
-  if (base >= nblocks) return;  // whole blocks only
-  const uint32_t tid = threadIdx.x;
-  const uint32_t b0 = base + tid * SCAN_PER;
-  uint32_t v[SCAN_PER];
-  uint32_t sum = 0;
-#pragma unroll
-  for (int k = 0; k < SCAN_PER; ++k) {
-    v[k] = b0 + k < nblocks ? counts[b0 + k] : 0u;
-    sum += v[k];
-  }
-  part[tid] = sum;
-  __syncthreads();
-  block_inclusive_scan(part);
-  uint32_t run = tid ? part[tid - 1] : 0u;
-#pragma unroll
-  for (int k = 0; k < SCAN_PER; ++k) {
-    if (b0 + k < nblocks) offsets[b0 + k] = run;
-    run += v[k];
-  }
-  if (tid == SCAN_THREADS - 1) chunk[blockIdx.x] = part[SCAN_THREADS - 1];
-}
-
-__global__ void __launch_bounds__(SCAN_THREADS)
-k_scan_top(const unsigned* __restrict__ count_ptr, uint32_t* __restrict__ chunk,
-           unsigned int* total, unsigned long long* segments, unsigned* fetch) {
-  __shared__ uint32_t part[SCAN_THREADS];
-  const uint32_t tid = threadIdx.x;
-  const uint32_t nblocks = (*count_ptr + BLOCK - 1) / BLOCK;
-  const uint32_t nchunks = (nblocks + SCAN_CHUNK - 1) / SCAN_CHUNK;
-  if (tid == 0) {
-    *segments += *count_ptr;
-    fetch[0] = fetch[1] = 0;  // tail-block counters of the next trace and shade
-  }
-  const uint32_t v = tid < nchunks ? chunk[tid] : 0u;
-  part[tid] = v;
-  __syncthreads();
-  block_inclusive_scan(part);
-  if (tid < nchunks) chunk[tid] = part[tid] - v;
-  if (tid == SCAN_THREADS - 1) *total = part[SCAN_THREADS - 1];
-}
-
-// Entry q of the next list: the q-th slot (in list order) that wrote a ray.
-// Same block partition as k_shade.
-template <bool LOOP>
-__global__ void __launch_bounds__(BLOCK)
-k_scatter(const uint32_t* __restrict__ list, const unsigned* __restrict__ count_ptr,
-          const uint8_t* __restrict__ emitted, const uint32_t* __restrict__ offsets,
-          const uint32_t* __restrict__ chunk, uint32_t* __restrict__ next) {
-  __shared__ uint32_t wcount[WAVES];
-  const uint32_t count = *count_ptr;
-  const uint32_t b_end = LOOP ? count : min(count, (blockIdx.x + 1) * BLOCK);
-  for (uint32_t b = blockIdx.x; b * BLOCK < b_end; b += gridDim.x) {  // whole logical blocks
-    const uint32_t q = b * BLOCK + threadIdx.x;
-    const bool live = q < count;
-    const uint32_t slot = live ? slot_of(list, q) : 0;
-    const bool pred = live && emitted[slot];
-    const uint64_t m = __ballot(pred);
-    const uint32_t w = threadIdx.x / 64;
-    if (lane_id() == 0) wcount[w] = (uint32_t)__popcll(m);
-    __syncthreads();
-    uint32_t base = offsets[b] + chunk[b / SCAN_CHUNK];
-    for (uint32_t i = 0; i < w; ++i) base += wcount[i];
-    const uint64_t below = m & ((1ull << lane_id()) - 1ull);
-    if (pred) next[base + (uint32_t)__popcll(below)] = slot;
-    __syncthreads();  // wcount is reused by the next logical block
-  }
-}
-
 #include "ssolh_fp32.hpp"
-#include "ssolh_render.hpp"
+#include "ssolh_path.hpp"
 
-// First work list: slots [0, n) in order, and its length
-__global__ void k_iota(uint32_t* __restrict__ list, uint32_t n, unsigned* __restrict__ count) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) list[i] = i;
-  if (i == 0) *count = n;
-}
+#include "ssolh_render.hpp"
 
 // Slot order of the first realisations by (sun, start instance). The
 // realisations are drawn at random over the field, so in realisation order a
@@ -2408,10 +1597,6 @@ struct ssolh_context {
   hipStream_t stream = nullptr;
   void* scratch = nullptr;  // this device's copy of the scratch array
   hipEvent_t ev[4] = {};
-  // graph drain: the list length after each of two replays in flight, in
-  // pinned host memory, and the events that mark it copied
-  hipEvent_t gev[2] = {};
-  unsigned* pinned = nullptr;
   // scene
   std::vector<DevBuf> scene_bufs;
   DScene scn{};
@@ -2420,22 +1605,7 @@ struct ssolh_context {
   uint64_t nprim = 0;
   uint32_t stack_depth = MAX_STACK;  // traversal stack bound of the scene's 4-wide nodes
   uint32_t lds_stack_cap = 0;        // 16, 24 or 32: LDS stack entries at most (0: MAX_STACK)
-  // The pending keys of every slot are NONE when a solve starts: a solve
-  // that drains leaves them so (each finished path clears its own), so they
-  // are cleared only when the path state's layout changed since the last
-  // solve that drained (state buffer, slots, entries, form) or it came from
-  // the scratch array.
-  struct KeysLayout {
-    void* state;
-    uint64_t slots;
-    uint32_t npend;
-    bool fp32;
-    bool operator==(const KeysLayout& o) const {
-      return state == o.state && slots == o.slots && npend == o.npend && fp32 == o.fp32;
-    }
-  };
-  KeysLayout keys_layout{};
-  bool keys_clean = false;
+  bool may_pend = false;  // a receiver may let light pass: paths keep pending entries
   float slack_scale = SLAB_SLACK;     // box-test slack of the scenes uploaded next
   // TLAS refit of moved instances: per-object boxes, the TLAS nodes by level
   // (deepest first) and the top copy's sources, all in scene_bufs
@@ -2455,9 +1625,10 @@ struct ssolh_context {
   DevBuf lbvh;
   DevBuf render;  // renderer work buffer (ssolh_render)
   // solve buffers
-  DevBuf start_sort;  // work bytes of the start-key sort of the first realisations
-  DevBuf state, rays, hits, lists[2], emitted, block_emits, block_offsets, scan_chunks, counters,
-      tallies, jobs, trace_ovf;
+  DevBuf start_sort;         // work bytes of the start-key sort
+  DevBuf queue[2], list;     // paths in flight, their list
+  DevBuf pend;               // pending entries
+  DevBuf counters, tallies, jobs, trace_ovf;
   // per-primitive log: keys, sorted keys, indices, sorted indices, values,
   // count, sort work (Tallies::log_*); log_sort, log_sidx, log_skey and
   // log_idx within it, log_sort_bytes of sort work
@@ -2476,8 +1647,6 @@ struct ssolh_context {
   uint64_t trk_cap = 0;
   uint32_t ninstances = 0;
   uint32_t njobs = 1;
-  PathState P{};
-  PathState32 P32{};
   const ShapeQ* shapeq = nullptr;  // per shape, in scene_bufs
   Tallies T{};
   size_t tally_bytes = 0;
@@ -2488,40 +1657,9 @@ struct ssolh_context {
   uint32_t iterations = 0;
   uint32_t wavefronts = 0;    // of the last solve
   uint32_t refilled = 0;
-  // grid of each looping kernel: its workgroups resident at once
-  std::vector<std::pair<const void*, uint32_t>> resident;
 };
 
 namespace {
-
-// Workgroups of each looping (graph-captured) kernel resident on the device
-// at once: occupancy per CU x CUs. A looping launch uses that grid, so every
-// workgroup starts at once and takes an equal share of the logical blocks;
-// with a larger grid the workgroups past the resident ones wait for whole
-// shares of others to end, and the tail runs on part of the chip.
-int init_resident_grids(ssolh_context* c, uint32_t cus) {
-  const void* fns[] = {
-      (const void*)k_trace<16, true>, (const void*)k_trace<24, true>,
-      (const void*)k_trace<MAX_STACK, true>,
-      (const void*)k_trace32<16, true>, (const void*)k_trace32<24, true>,
-      (const void*)k_trace32<MAX_STACK, true>,
-      (const void*)k_shade<false, false, true>, (const void*)k_shade<false, true, true>,
-      (const void*)k_shade<true, false, true>, (const void*)k_shade<true, true, true>,
-      (const void*)k_shade32<false, true>, (const void*)k_shade32<true, true>,
-      (const void*)k_scatter<true>};
-  for (const void* f : fns) {
-    int per_cu = 0;
-    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, BLOCK, 0));
-    c->resident.push_back({f, (uint32_t)std::max(per_cu, 1) * cus});
-  }
-  return 0;
-}
-
-uint32_t resident_grid(const ssolh_context* c, const void* f) {
-  for (const auto& e : c->resident)
-    if (e.first == f) return e.second;
-  return 1024;  // not reached: init_resident_grids lists every looping kernel
-}
 
 int dev_alloc(DevBuf& b, size_t bytes) {
   if (b.n >= bytes && b.p) return 0;
@@ -2777,12 +1915,6 @@ SSOLH_API int ssolh_create(int device, ssolh_context** out) {
   c->scratch = scratch_ptr;
   HIP_TRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
   for (auto& e : c->ev) HIP_TRY(hipEventCreate(&e));
-  for (auto& e : c->gev) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  HIP_TRY(hipHostMalloc((void**)&c->pinned, 2 * sizeof(unsigned), hipHostMallocDefault));
-  if (int r = init_resident_grids(c, (uint32_t)prop.multiProcessorCount)) {
-    ssolh_destroy(c);
-    return r;
-  }
   *out = c;
   return 0;
 }
@@ -2792,15 +1924,12 @@ SSOLH_API int ssolh_destroy(ssolh_context* c) {
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   free_scene(c);
-  for (DevBuf* b : {&c->state, &c->rays, &c->hits, &c->lists[0], &c->lists[1], &c->emitted,
-                    &c->block_emits, &c->block_offsets, &c->scan_chunks, &c->counters, &c->tallies,
-                    &c->jobs, &c->start_sort, &c->trace_ovf, &c->lbvh, &c->render, &c->plog,
+  for (DevBuf* b : {&c->start_sort, &c->queue[0], &c->queue[1], &c->list, &c->pend, &c->counters,
+                    &c->tallies, &c->jobs, &c->trace_ovf, &c->lbvh, &c->render, &c->plog,
                     &c->adj_state, &c->adj_in, &c->adj_grad, &c->trk_vtx, &c->trk_type,
                     &c->trk_seq, &c->trk_count, &c->trk_pos})
     if (b->p) (void)hipFree(b->p);
   for (auto& e : c->ev) if (e) (void)hipEventDestroy(e);
-  for (auto& e : c->gev) if (e) (void)hipEventDestroy(e);
-  if (c->pinned) (void)hipHostFree(c->pinned);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
   return 0;
@@ -2967,6 +2096,18 @@ SSOLH_API int ssolh_scene_upload(ssolh_context* c, const struct ssolh_scene* s) 
   c->inst_object.resize(s->ninstances);
   for (uint32_t i = 0; i < s->ninstances; ++i) c->inst_object[i] = s->instances[i].object;
   HIP_TRY(hipStreamSynchronize(c->stream));  // the host arrays may go after return
+  // pending entries are kept by paths that a receiver does not end: not
+  // where every receiving side absorbs all light
+  c->may_pend = false;
+  for (const IssInfo& x : iss) {
+    if (x.receiver < 0) continue;
+    for (uint32_t side : {SSOL_FRONT_, SSOL_BACK_}) {
+      const ssolh_material& m = s->materials[side == SSOL_FRONT_ ? x.mtl_front : x.mtl_back];
+      const bool black = (m.type == SSOLH_MTL_MATTE || m.type == SSOLH_MTL_MIRROR) &&
+                         m.reflectivity == 0;
+      if ((x.receiver_mask & side) && !black) c->may_pend = true;
+    }
+  }
   c->has_scene = true;
   ++c->n_uploads;
   return 0;
@@ -3131,14 +2272,14 @@ SSOLH_API int ssolh_render(ssolh_context* c, const struct ssolh_render_args* a, 
       if (iter >= 100000) { set_err("ssolh_render: paths did not end"); return SSOLH_ERR_LIMIT; }
       const uint32_t tb = (n + BLOCK - 1) / BLOCK;
       if (lds_stack == 16)
-        k_trace<16, false><<<tb, BLOCK, 0, c->stream>>>(c->scn, lists[cur], cnt + cur, rays, hits,
-                                                       cnt + 2, ovf);
+        k_trace<16><<<tb, BLOCK, 0, c->stream>>>(c->scn, lists[cur], cnt + cur, rays, hits,
+                                                ovf);
       else if (lds_stack == 24)
-        k_trace<24, false><<<tb, BLOCK, 0, c->stream>>>(c->scn, lists[cur], cnt + cur, rays, hits,
-                                                       cnt + 2, ovf);
+        k_trace<24><<<tb, BLOCK, 0, c->stream>>>(c->scn, lists[cur], cnt + cur, rays, hits,
+                                                ovf);
       else
-        k_trace<MAX_STACK, false><<<tb, BLOCK, 0, c->stream>>>(c->scn, lists[cur], cnt + cur,
-                                                              rays, hits, cnt + 2, ovf);
+        k_trace<MAX_STACK><<<tb, BLOCK, 0, c->stream>>>(c->scn, lists[cur], cnt + cur,
+                                                              rays, hits, ovf);
       HIP_TRY(hipGetLastError());
       HIP_TRY(hipMemsetAsync(cnt + (cur ^ 1), 0, sizeof(unsigned), c->stream));
       k_render_shade<<<blocks, BLOCK, 0, c->stream>>>(c->scn, rp, st, rays, hits, pix,
@@ -3175,11 +2316,7 @@ SSOLH_API int ssolh_test_scene_counters(ssolh_context* c, uint32_t* uploads, uin
 
 namespace {
 
-// One solve over `njobs` suns (njobs == 1: the scene's sun). Realisation
-// ids [0, N) map to jobs through job_first. graph_iters > 0 captures that
-// many iterations (rounded up to even) into a HIP graph replayed until the
-// work list is empty; 0 runs the iterations from the host one by one.
-// Host description of an adjoint solve (host pointers)
+// Host description of a tracked and of an adjoint solve (host pointers)
 struct TrackHost {
   double sun_len, inf_len;
   uint64_t cap;
@@ -3193,16 +2330,18 @@ struct AdjHost {
   double d_total;
 };
 
+// One solve over `njobs` suns (njobs == 1: the scene's sun). Realisation
+// ids [0, N) map to jobs through job_first.
 int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, uint64_t counter,
               bool fp32, uint32_t path_slots, uint32_t npend, uint32_t njobs,
-              const uint64_t* job_first_h, const ssolh_sun* job_suns_h, uint32_t graph_iters,
+              const uint64_t* job_first_h, const ssolh_sun* job_suns_h,
               const AdjHost* adj = nullptr, const TrackHost* trk = nullptr,
               Arena* arena = nullptr) {
   // buffers come from the device allocator, or all from the arena
   auto alloc = [&](DevBuf& b, size_t bytes) -> int {
     return arena ? arena_take(*arena, b, bytes) : dev_alloc(b, bytes);
   };
-  if (arena && (adj || trk || job_suns_h || graph_iters)) {
+  if (arena && (adj || trk || job_suns_h)) {
     set_err("ssolh_solve_noalloc: plain single-sun solves driven from the host only");
     return SSOLH_ERR_ARG;
   }
@@ -3211,8 +2350,7 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
     set_err("ssolh_solve_tracked: paths are recorded by plain FP64 solves only");
     return SSOLH_ERR_ARG;
   }
-  if (trk) graph_iters = 0;
-  else c->trk_paths = 0;  // the recorded paths belong to the last solve only
+  if (!trk) c->trk_paths = 0;  // the recorded paths belong to the last solve only
   if (npend > MAX_PEND) { set_err("ssolh_solve: at most %d pending entries", MAX_PEND); return SSOLH_ERR_LIMIT; }
   // Tally layout: each tally is striped over up to 256 copies while its
   // stripes hold at most 2^21 doubles; from the scratch array every stripe
@@ -3244,33 +2382,45 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
             "scratch array", tally_bytes, arena->size / 2);
     return SSOLH_ERR_LIMIT;
   }
-  // Wavefront width. By default every realisation is in flight at once when
-  // 2/5 of the device memory holds their state: the realisations then start
-  // together and each iteration traces one generation of rays (shadow rays,
-  // first reflections, ...), which keeps the waves coherent; larger solves
-  // run as many as fit, each slot taking its next realisation in place.
-  uint64_t slots64 = path_slots;
-  const size_t per_slot = (fp32 ? 5 * sizeof(float4) + 3 * sizeof(uint4)
-                               : sizeof(double2) + 3 * sizeof(double4) + 3 * sizeof(uint4)) +
-                          (size_t)npend * 2 * (sizeof(uint32_t) + 10 * (fp32 ? sizeof(float) : sizeof(double))) +
-                          (fp32 ? sizeof(RayRec32) + sizeof(HitRec32) : sizeof(RayRec) + sizeof(HitRec)) +
-                          2 * sizeof(uint32_t) + 1 + (adj ? sizeof(double4) + sizeof(uint32_t) : 0) +
+  // Wavefront width. By default every realisation of the solve is in flight
+  // at once, in start-instance order, when 2/5 of the device memory holds
+  // what a realisation keeps there: its place in the order, its places in the
+  // path queues and, in scenes whose receivers let light pass, its pending
+  // entries. Larger solves run as many as fit at a time.
+  const uint32_t npend_asked = npend;
+  if (!c->may_pend) npend = 0;
+  const size_t real = fp32 ? sizeof(float) : sizeof(double);
+  const size_t planes = fp32 ? RAY_PLANES32 + STATE_PLANES32 : RAY_PLANES64 + STATE_PLANES64;
+  TOvf ovf{nullptr, 0, c->stack_depth > START_STACK ? c->stack_depth - START_STACK : 0u};
+  const size_t per_slot = 2 * sizeof(uint32_t) + 2 * planes * 16 + ovf.extra * sizeof(uint32_t) +
+                          (size_t)npend * 2 * (sizeof(uint32_t) + 10 * real) +
+                          (adj ? sizeof(double4) + sizeof(uint32_t) : 0) +
                           (trk ? sizeof(uint32_t) + sizeof(double4) : 0);
-  if (!slots64 && arena) {
-    // from the scratch array: what is left beside the tallies, the
-    // per-block scan arrays, counters and start-instance histogram
+  uint64_t slots64 = path_slots;
+  if (arena) {
+    // An asked width is refused past what the array holds of slots with a
+    // ray, a hit, a path record and pending entries each, whatever the scene
+    // needs of these. The width taken is what is left beside the tallies, the
+    // sort's work bytes and the alignment of the parts.
+    const size_t most_slot = fp32 ? 233 + 88 * (size_t)npend_asked : 281 + 168 * (size_t)npend_asked;
+    const uint64_t asked = std::min<uint64_t>(path_slots, N);
+    if (asked > (arena->size - tally_bytes) / most_slot) {
+      set_err("ssolh_solve_noalloc: %llu path slots do not fit beside the tallies in the scratch "
+              "array", (unsigned long long)asked);
+      return SSOLH_ERR_LIMIT;
+    }
     size_t sort_bytes = 0;
     const uint64_t most = std::min<uint64_t>(std::min<uint64_t>(N, arena->size / per_slot), 1u << 28);
     HIP_TRY(start_sort_bytes((uint32_t)most, start_key_bits((uint64_t)njobs * c->ninstances),
                              c->stream, sort_bytes));
     const size_t fixed = tally_bytes + (sort_bytes + 255) / 256 * 256 + (64u << 10);
     const size_t rest = arena->size > fixed ? arena->size - fixed : 0;
-    slots64 = rest / (per_slot + 1) / BLOCK * BLOCK;  // + 8 B of per-block counts per block
+    slots64 = rest / per_slot / BLOCK * BLOCK;
     if (slots64 < BLOCK) {
       set_err("ssolh_solve_noalloc: no path slot fits beside the tallies in the scratch array");
       return SSOLH_ERR_LIMIT;
     }
-    if (slots64 > N) slots64 = N;
+    if (path_slots) slots64 = std::min<uint64_t>(slots64, path_slots);
   }
   if (!slots64) {
     size_t free_b = 0, total_b = 0;
@@ -3280,7 +2430,7 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
     // and within what is free now (this context's own solve buffers count
     // as free: they are reallocated), when other work holds device memory
     size_t held = 0;
-    for (const DevBuf* b : {&c->state, &c->rays, &c->hits, &c->lists[0], &c->lists[1], &c->emitted,
+    for (const DevBuf* b : {&c->queue[0], &c->queue[1], &c->list, &c->pend, &c->trace_ovf,
                             &c->adj_state, &c->trk_seq})
       held += b->n;
     const uint64_t fit_free = (uint64_t)((free_b + held) / 10 * 9) / per_slot;
@@ -3290,82 +2440,51 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
   slots64 = (slots64 + BLOCK - 1) / BLOCK * BLOCK;
   if (slots64 > (1ull << 28)) { set_err("ssolh_solve: at most 2^28 path slots"); return SSOLH_ERR_LIMIT; }
   const uint32_t slots = (uint32_t)slots64;
-  const uint32_t max_blocks = slots / BLOCK;
-
-  // path state: arrays of 16- or 32-byte records and the pending entries,
-  // each array starting on a 256-byte boundary
   const size_t n = slots;
-  const size_t real = fp32 ? sizeof(float) : sizeof(double);
-  const size_t pend_keys = npend * n * sizeof(uint32_t), pend_vals = npend * n * 10 * real;
-  std::vector<size_t> sizes;
-  if (fp32)
-    sizes = {n * sizeof(float4), n * sizeof(float4), n * sizeof(float4), n * sizeof(float4),
-             n * sizeof(float4), n * sizeof(uint4), n * sizeof(uint4), n * sizeof(uint4),
-             pend_keys, pend_keys, pend_vals, pend_vals};
-  else
-    sizes = {n * sizeof(double2), n * sizeof(double4), n * sizeof(double4), n * sizeof(double4),
-             n * sizeof(uint4), n * sizeof(uint4), n * sizeof(uint4), pend_keys, pend_keys,
-             pend_vals, pend_vals};
-  size_t bytes_state = 0;
-  for (size_t sz : sizes) bytes_state += (sz + 255) / 256 * 256;
-  int r = alloc(c->state, bytes_state);
-  if (r) return r;
-  {
-    char* p = (char*)c->state.p;
-    std::vector<void*> arr(sizes.size());
-    for (size_t i = 0; i < sizes.size(); ++i) { arr[i] = p; p += (sizes[i] + 255) / 256 * 256; }
-    if (fp32) {
-      c->P32.pos = (float4*)arr[0];
-      c->P32.prev_init = (float4*)arr[1];
-      c->P32.out_in0 = (float4*)arr[2];
-      c->P32.nrm_t = (float4*)arr[3];
-      c->P32.pend_cos = (float4*)arr[4];
-      c->P32.meta = (uint4*)arr[5];
-      c->P32.cur = (uint4*)arr[6];
-      c->P32.misc = (uint4*)arr[7];
-      c->P32.pkey = (uint32_t*)arr[8];
-      c->P32.qkey = (uint32_t*)arr[9];
-      c->P32.pval = (float*)arr[10];
-      c->P32.qval = (float*)arr[11];
-    } else {
-      c->P.cst = (double2*)arr[0];
-      c->P.pw = (double4*)arr[1];
-      c->P.nrm = (double4*)arr[2];
-      c->P.pend = (double4*)arr[3];
-      c->P.st = (uint4*)arr[4];
-      c->P.sm = (uint4*)arr[5];
-      c->P.aux = (uint4*)arr[6];
-      c->P.pkey = (uint32_t*)arr[7];
-      c->P.qkey = (uint32_t*)arr[8];
-      c->P.pval = (double*)arr[9];
-      c->P.qval = (double*)arr[10];
-    }
+
+  // With fewer slots than realisations the solve runs in chunks of `slots`
+  // realisations, one after the other. Each is put in start-instance order
+  // when there is something to order by (more than one sun or sampled
+  // instance); otherwise realisation s of a chunk takes slot s, and the
+  // chunks count as one wavefront whose slots take further realisations.
+  const uint64_t nkeys = (uint64_t)njobs * c->ninstances;
+  const bool orderable = (uint64_t)njobs * c->nsamp > 1 && nkeys <= (1u << 24);
+  const bool refill = slots < N && !orderable;
+
+  // start order: keys and indices before and after their sort, in the queue
+  // that is not written before they have been read
+  const uint32_t key_bits = start_key_bits(nkeys);
+  const size_t part = (n + 63) / 64 * 64;  // 256-byte aligned parts
+  size_t sort_bytes = 0;
+  int r = 0;
+  if (orderable) {
+    HIP_TRY(start_sort_bytes(slots, key_bits, c->stream, sort_bytes));
+    if ((r = alloc(c->start_sort, sort_bytes))) return r;
   }
-  {
-    const ssolh_context::KeysLayout lay{c->state.p, n, npend, fp32};
-    const bool clean = !arena && c->keys_clean && c->keys_layout == lay;
-    c->keys_clean = false;  // until this solve drains
-    c->keys_layout = lay;
-    if (!clean && npend) {
-      HIP_TRY(hipMemsetAsync(fp32 ? c->P32.pkey : c->P.pkey, 0xFF, pend_keys, c->stream));
-      HIP_TRY(hipMemsetAsync(fp32 ? c->P32.qkey : c->P.qkey, 0xFF, pend_keys, c->stream));
-    }
+  // path queues, the list of places in the one being read, the waves' counts
+  // of paths written and their scan
+  for (int i = 0; i < 2; ++i)
+    if ((r = alloc(c->queue[i], part * planes * 16))) return r;
+  const uint32_t waves = slots / 64, chunks = (waves + SCAN_CHUNK - 1) / SCAN_CHUNK;
+  if ((r = alloc(c->list, (n + 2 * waves + chunks) * sizeof(uint32_t)))) return r;
+  uint32_t* const list = (uint32_t*)c->list.p;
+  uint32_t *const wave_n = list + n, *const wave_off = wave_n + waves,
+           *const wave_chunk = wave_off + waves;
+  Pending W{};
+  W.npend = npend;
+  if (npend) {
+    const size_t keys = npend * n * sizeof(uint32_t), vals = npend * n * 10 * real;
+    if ((r = alloc(c->pend, 2 * keys + 2 * vals))) return r;
+    char* p = (char*)c->pend.p;  // each part a multiple of 128 * 4 bytes
+    W.pkey = (uint32_t*)p;
+    W.qkey = (uint32_t*)(p + keys);
+    W.pval = p + 2 * keys;
+    W.qval = p + 2 * keys + vals;
   }
-  if ((r = alloc(c->rays, n * (fp32 ? sizeof(RayRec32) : sizeof(RayRec))))) return r;
-  if ((r = alloc(c->hits, n * (fp32 ? sizeof(HitRec32) : sizeof(HitRec))))) return r;
-  for (int i = 0; i < 2; ++i) if ((r = alloc(c->lists[i], n * sizeof(uint32_t)))) return r;
-  if ((r = alloc(c->emitted, n))) return r;
-  if ((r = alloc(c->block_emits, max_blocks * sizeof(uint32_t)))) return r;
-  if ((r = alloc(c->block_offsets, max_blocks * sizeof(uint32_t)))) return r;
-  if ((r = alloc(c->scan_chunks, ((max_blocks + SCAN_CHUNK - 1) / SCAN_CHUNK) * sizeof(uint32_t))))
-    return r;
-  if ((r = alloc(c->counters, sizeof(Counters) + 4 * sizeof(unsigned)))) return r;
-  // traversal stack entries past the LDS ones (scenes whose bound exceeds
-  // MAX_STACK), per work-list position
-  const uint32_t lds_stack = trace_lds_stack(c);
-  TOvf ovf{nullptr, slots, 0};
-  if (c->stack_depth > lds_stack) {
-    ovf.extra = c->stack_depth - lds_stack;
+  if ((r = alloc(c->counters, sizeof(Counters)))) return r;
+  // traversal stack entries past the LDS ones, per lane of a launch
+  if (ovf.extra) {
+    ovf.stride = slots;
     if ((r = alloc(c->trace_ovf, n * ovf.extra * sizeof(uint32_t)))) return r;
     ovf.base = (uint32_t*)c->trace_ovf.p;
   }
@@ -3450,7 +2569,7 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
   c->T.njobs = njobs;
   c->njobs = njobs;
   HIP_TRY(hipMemsetAsync(c->tallies.p, 0, tally_bytes, c->stream));
-  HIP_TRY(hipMemsetAsync(c->counters.p, 0, sizeof(Counters) + 4 * sizeof(unsigned), c->stream));
+  HIP_TRY(hipMemsetAsync(c->counters.p, 0, sizeof(Counters), c->stream));
   // per-primitive log: room for one record per realisation, at most
   // LOG_MAX_RECORDS (12.9 GB); none from the scratch array
   c->T.log_key = nullptr;
@@ -3494,7 +2613,7 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
     }
   }
   // Sums the logged records into the per-primitive tally and empties the
-  // log (outside graph capture: the stream is the solve's)
+  // log
   auto log_flush = [&]() -> int {
     if (!c->T.log_cap) return 0;
     unsigned long long n = 0;
@@ -3532,286 +2651,126 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
                             : nullptr;
 
   Counters* ctr = (Counters*)c->counters.p;
-  unsigned* cnt = (unsigned*)((char*)c->counters.p + sizeof(Counters));  // [2] list lengths
-  // tail-block counters of the looping trace and shade kernels (zeroed with
-  // the counters, then by every k_scan_top)
-  unsigned* fetch = cnt + 2;
-  uint32_t* lists[2] = {(uint32_t*)c->lists[0].p, (uint32_t*)c->lists[1].p};
-  uint8_t* emitted = (uint8_t*)c->emitted.p;
-  uint32_t* block_emits = (uint32_t*)c->block_emits.p;
-  uint32_t* block_offsets = (uint32_t*)c->block_offsets.p;
-  uint32_t* scan_chunks = (uint32_t*)c->scan_chunks.p;
+  PathArgs args{};
+  args.S = c->scn;
+  args.SQ = c->shapeq;
+  args.prm = prm;
+  args.T = c->T;
+  args.W = W;
+  args.C = ctr;
+  args.A = A;
+  args.K = K;
+  args.ovf = ovf;
 
-  // With fewer slots than realisations and something to order by (more than
-  // one sun or sampled instance), the solve runs in chunks of `slots`
-  // realisations, each all in flight and in start-instance order, instead of
-  // refilling slots in place (100-paraboloid field at 2^20 slots: 449 -> 629
-  // Mpaths/s; its 512-sun sweep, 51,712 keys: 1,680 -> 2,290).
-  const uint64_t nkeys = (uint64_t)njobs * c->ninstances;
-  const bool orderable = (uint64_t)njobs * c->nsamp > 1 && nkeys <= (1u << 24);
-  const bool chunked = slots < N && orderable;
+  args.wave_in = args.wave_out = wave_n;
+  args.in_n = &ctr->left;
 
-  // one iteration: trace, shade, compaction of list i into list i^1
-  auto iteration = [&](int i, uint32_t blocks) -> int {
-    // blocks: logical blocks of the list (of its largest length under graph
-    // capture). The host loop launches one workgroup per logical block; a
-    // captured iteration launches each kernel's resident grid, whose
-    // workgroups loop over the logical blocks, however long or short the
-    // list turns out to be
-    const bool loop = graph_iters != 0;
-    auto grid_of = [&](const void* f) {
-      return loop ? std::min<uint32_t>(blocks, resident_grid(c, f)) : blocks;
-    };
-    const uint32_t* list = lists[i];
-    const unsigned* count = cnt + i;
-    const bool refill = slots < N && !chunked;
-    if (fp32) {
-      RayRec32* r32 = (RayRec32*)c->rays.p;
-      HitRec32* h32 = (HitRec32*)c->hits.p;
-      auto launch = [&](auto kernel) {
-        kernel<<<grid_of((const void*)kernel), BLOCK, 0, c->stream>>>(c->scn, c->shapeq, list,
-                                                                     count, r32, h32, fetch, ovf);
-      };
-      if (lds_stack == 16)
-        loop ? launch(k_trace32<16, true>) : launch(k_trace32<16, false>);
-      else if (lds_stack == 24)
-        loop ? launch(k_trace32<24, true>) : launch(k_trace32<24, false>);
-      else
-        loop ? launch(k_trace32<MAX_STACK, true>) : launch(k_trace32<MAX_STACK, false>);
-    } else {
-      RayRec* r64 = (RayRec*)c->rays.p;
-      HitRec* h64 = (HitRec*)c->hits.p;
-      auto launch = [&](auto kernel) {
-        kernel<<<grid_of((const void*)kernel), BLOCK, 0, c->stream>>>(c->scn, list, count, r64,
-                                                                     h64, fetch, ovf);
-      };
-      if (lds_stack == 16)
-        loop ? launch(k_trace<16, true>) : launch(k_trace<16, false>);
-      else if (lds_stack == 24)
-        loop ? launch(k_trace<24, true>) : launch(k_trace<24, false>);
-      else
-        loop ? launch(k_trace<MAX_STACK, true>) : launch(k_trace<MAX_STACK, false>);
-    }
-    HIP_TRY(hipGetLastError());
-    if (!graph_iters) HIP_TRY(hipEventRecord(c->ev[2], c->stream));
-    if (fp32) {
-      const Shade32Args args{c->scn,     c->shapeq, c->P32, prm, c->T, list, count,
-                             (RayRec32*)c->rays.p, (const HitRec32*)c->hits.p, emitted,
-                             block_emits, ctr, fetch + 1};
-      auto launch = [&](auto kernel) {
-        kernel<<<grid_of((const void*)kernel), BLOCK, 0, c->stream>>>(args);
-      };
-      if (refill) loop ? launch(k_shade32<true, true>) : launch(k_shade32<true, false>);
-      else loop ? launch(k_shade32<false, true>) : launch(k_shade32<false, false>);
-    } else {
-      const ShadeArgs args{c->scn,  c->P,     prm,         c->T, list, count, (RayRec*)c->rays.p,
-                           (const HitRec*)c->hits.p, emitted, block_emits, ctr,  A,    K,
-                           fetch + 1};
-      auto launch = [&](auto kernel) {
-        kernel<<<grid_of((const void*)kernel), BLOCK, 0, c->stream>>>(args);
-      };
-      if (A.grad && refill)
-        loop ? launch(k_shade<true, true, true>) : launch(k_shade<true, true, false>);
-      else if (A.grad)
-        loop ? launch(k_shade<true, false, true>) : launch(k_shade<true, false, false>);
-      else if (refill)
-        loop ? launch(k_shade<false, true, true>) : launch(k_shade<false, true, false>);
-      else
-        loop ? launch(k_shade<false, false, true>) : launch(k_shade<false, false, false>);
-    }
-    HIP_TRY(hipGetLastError());
-    if (!graph_iters) HIP_TRY(hipEventRecord(c->ev[3], c->stream));
-    k_scan_chunks<<<(blocks + SCAN_CHUNK - 1) / SCAN_CHUNK, SCAN_THREADS, 0, c->stream>>>(
-        block_emits, count, block_offsets, scan_chunks);
-    HIP_TRY(hipGetLastError());
-    k_scan_top<<<1, SCAN_THREADS, 0, c->stream>>>(count, scan_chunks, cnt + (i ^ 1), &ctr->segments,
-                                                  fetch);
-    HIP_TRY(hipGetLastError());
-    if (loop)
-      k_scatter<true><<<grid_of((const void*)k_scatter<true>), BLOCK, 0, c->stream>>>(
-          list, count, emitted, block_offsets, scan_chunks, lists[i ^ 1]);
-    else
-      k_scatter<false><<<blocks, BLOCK, 0, c->stream>>>(list, count, emitted, block_offsets,
-                                                        scan_chunks, lists[i ^ 1]);
+  auto launch = [&](uint32_t blocks, auto k32, auto k64, auto kadj, auto ktrk) -> int {
+    auto go = [&](auto kernel) { kernel<<<blocks, BLOCK, 0, c->stream>>>(args); };
+    fp32 ? go(k32) : adj ? go(kadj) : trk ? go(ktrk) : go(k64);
     HIP_TRY(hipGetLastError());
     return 0;
   };
+  auto start = [&](uint32_t count) {
+    return launch((count + BLOCK - 1) / BLOCK, k_start<F32, false, false>,
+                  k_start<F64, false, false>, k_start<F64, true, false>,
+                  k_start<F64, false, true>);
+  };
+  // few paths run through, unless their entries could fill the log
+  auto run_through = [&](uint32_t count) {
+    return count <= RUN_THROUGH && (!c->T.log_cap || count <= c->T.log_cap);
+  };
+  auto resume = [&](uint32_t count) {
+    const uint32_t blocks = (count + BLOCK - 1) / BLOCK;
+    return run_through(count)
+               ? launch(blocks, k_resume<F32, false, false, true>,
+                        k_resume<F64, false, false, true>, k_resume<F64, true, false, true>,
+                        k_resume<F64, false, true, true>)
+               : launch(blocks, k_resume<F32, false, false, false>,
+                        k_resume<F64, false, false, false>, k_resume<F64, true, false, false>,
+                        k_resume<F64, false, true, false>);
+  };
 
-  float ms_trace = 0, ms_shade = 0;
-  HIP_TRY(hipEventRecord(c->ev[0], c->stream));
-
-  // The first realisations of a wavefront, first .. first + count - 1, fill
-  // slots [0, count) (list 0 is 0..count-1): in start-instance order when
-  // no slot is refilled (a chunk, or every realisation in flight; refilled
-  // slots take realisations r + slots, which in id order stay on one sun per
-  // wave and in this order would not). The keys and indices before and
-  // after the sort take the hit records, the order the second work list,
-  // neither of which is used before the first trace.
-  auto start = [&](uint64_t first, uint32_t count) -> int {
-    k_iota<<<(count + 255) / 256, 256, 0, c->stream>>>(lists[0], count, cnt);
-    HIP_TRY(hipGetLastError());
-    const uint32_t* order = nullptr;
-    if (count && (chunked || first + count == N) && orderable) {
-      const uint32_t bits = start_key_bits(nkeys), gg = (count + 255) / 256;
-      size_t sort_bytes = 0;
-      HIP_TRY(start_sort_bytes(count, bits, c->stream, sort_bytes));
-      if (int e = alloc(c->start_sort, sort_bytes)) return e;
-      const size_t part = (size_t)(count + 63) / 64 * 64;  // 256-byte aligned parts
-      uint32_t* key = (uint32_t*)c->hits.p;
-      uint32_t* skey = key + part;
-      uint32_t* idx = skey + part;
-      if (fp32)
-        k_start_keys<true><<<gg, 256, 0, c->stream>>>(c->scn, prm, first, count, c->ninstances,
-                                                       key, idx);
-      else
-        k_start_keys<false><<<gg, 256, 0, c->stream>>>(c->scn, prm, first, count, c->ninstances,
-                                                        key, idx);
-      HIP_TRY(hipGetLastError());
-      HIP_TRY(hipcub::DeviceRadixSort::SortPairs(c->start_sort.p, sort_bytes, key, skey, idx,
-                                                 lists[1], (int)count, 0, (int)bits, c->stream));
-      order = lists[1];
-    }
-    const uint32_t gb = (count + BLOCK - 1) / BLOCK;
+  // The realisations first .. first + count - 1 in start-instance order:
+  // drawn keys, then a stable radix sort of (key, index)
+  auto order_starts = [&](uint64_t first, uint32_t count) -> int {
+    uint32_t* key = (uint32_t*)c->queue[1].p;
+    uint32_t *skey = key + part, *idx = skey + part, *order = idx + part;
+    const uint32_t gg = (count + 255) / 256;
     if (fp32)
-      k_generate32<<<gb, BLOCK, 0, c->stream>>>(c->scn, c->shapeq, c->P32, prm, c->T,
-                                                (RayRec32*)c->rays.p, first, count, order);
-    else if (A.grad)
-      k_generate<true><<<gb, BLOCK, 0, c->stream>>>(c->scn, c->P, prm, c->T, (RayRec*)c->rays.p,
-                                                    first, count, A, K, order);
+      k_start_keys<true><<<gg, 256, 0, c->stream>>>(c->scn, prm, first, count, c->ninstances, key,
+                                                     idx);
     else
-      k_generate<false><<<gb, BLOCK, 0, c->stream>>>(c->scn, c->P, prm, c->T, (RayRec*)c->rays.p,
-                                                     first, count, A, K, order);
+      k_start_keys<false><<<gg, 256, 0, c->stream>>>(c->scn, prm, first, count, c->ninstances,
+                                                      key, idx);
     HIP_TRY(hipGetLastError());
+    size_t sb = sort_bytes;
+    HIP_TRY(hipcub::DeviceRadixSort::SortPairs(c->start_sort.p, sb, key, skey, idx, order,
+                                               (int)count, 0, (int)key_bits, c->stream));
+    args.order = order;
     return 0;
   };
 
-  // iterations of the whole solve (reported) and of the current wavefront
-  // (bounded: a wavefront drains within its deepest path, which roulette
-  // ends with probability 1 - 2^-k after 16k bounces past depth 65)
-  uint32_t iter = 0, wave_iter = 0;
-  constexpr uint32_t MAX_WAVE_ITER = 1000000u;
-  // host-driven iterations until the list is empty
-  auto drain_host = [&](uint32_t count) -> int {
-    int cur = 0;
-    while (count) {
-      if (wave_iter >= MAX_WAVE_ITER) {
-        set_err("ssolh_solve: the wavefront did not drain after %u iterations", wave_iter);
-        return SSOLH_ERR_LIMIT;
-      }
-      HIP_TRY(hipEventRecord(c->ev[1], c->stream));
-      if (int e = iteration(cur, (count + BLOCK - 1) / BLOCK)) return e;
-      unsigned total = 0;
-      unsigned long long logged = 0;
-      HIP_TRY(hipMemcpyAsync(&total, cnt + (cur ^ 1), sizeof(total), hipMemcpyDeviceToHost, c->stream));
-      if (c->T.log_cap)
-        HIP_TRY(hipMemcpyAsync(&logged, c->T.log_n, sizeof(logged), hipMemcpyDeviceToHost, c->stream));
-      HIP_TRY(hipStreamSynchronize(c->stream));
-      float t1 = 0, t2 = 0;
-      (void)hipEventElapsedTime(&t1, c->ev[1], c->ev[2]);
-      (void)hipEventElapsedTime(&t2, c->ev[2], c->ev[3]);
-      ms_trace += t1;
-      ms_shade += t2;
-      if (total > count) {
-        set_err("ssolh_solve: work list grew from %u to %u entries", count, total);
-        return SSOLH_ERR_LIMIT;
-      }
-      cur ^= 1;
-      count = total;
-      ++iter;
-      ++wave_iter;
-      // past half full, the log is summed before it overflows into atomics
-      if (count && c->T.log_cap && logged >= c->T.log_cap / 2)
-        if (int e = log_flush()) return e;
-    }
-    return 0;
-  };
-
-  // graph of an even number of iterations: list 0 -> 1 -> 0 ...; every
-  // kernel reads its work count from device memory, so iterations past the
-  // end of the work are empty launches. Captured once, replayed for every
-  // chunk until its list is empty.
-  const uint32_t gi = (graph_iters + 1) & ~1u;
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  // graph replays until the list is empty, two in flight: the list length
-  // after replay k is copied to pinned memory and read while replay k+1
-  // runs, so the GPU does not wait for the host between replays; a replay
-  // past the end runs empty launches
-  auto drain_graph = [&](uint32_t count) -> int {
-    uint32_t launched = 0, seen = 0;
-    while (count) {
-      while (launched - seen < 2) {
-        if (wave_iter >= MAX_WAVE_ITER) {
-          set_err("ssolh_solve: the wavefront did not drain after %u iterations", wave_iter);
-          (void)hipStreamSynchronize(c->stream);
+  float ms_path = 0;
+  HIP_TRY(hipEventRecord(c->ev[0], c->stream));
+  for (uint64_t first = 0; first < N; first += slots) {
+    const uint32_t count = (uint32_t)std::min<uint64_t>(N - first, slots);
+    args.first = first;
+    args.count = count;
+    args.order = nullptr;
+    const bool wave = !refill || first == 0;
+    k_path_begin<<<1, 1, 0, c->stream>>>(ctr, wave);
+    HIP_TRY(hipGetLastError());
+    if (orderable) if ((r = order_starts(first, count))) return r;
+    HIP_TRY(hipEventRecord(c->ev[1], c->stream));
+    PathQ from{(uint4*)c->queue[1].p, slots}, to{(uint4*)c->queue[0].p, slots};
+    args.out = to;
+    if ((r = start(count))) return r;
+    // the paths that go on, from queue to queue, until a launch runs them
+    // through; a few start in the places where k_start left them
+    uint32_t going = count;
+    args.list = nullptr;
+    do {
+      if (!run_through(going)) {
+        const uint32_t w = (going + 63) / 64, ch = (w + SCAN_CHUNK - 1) / SCAN_CHUNK;
+        k_scan_chunks<<<ch, SCAN_THREADS, 0, c->stream>>>(wave_n, w, wave_off, wave_chunk);
+        HIP_TRY(hipGetLastError());
+        k_scan_top<<<1, SCAN_THREADS, 0, c->stream>>>(ch, wave_chunk, &ctr->left, ctr);
+        HIP_TRY(hipGetLastError());
+        k_queue_list<<<(w + 3) / 4, 256, 0, c->stream>>>(wave_n, w, wave_off, wave_chunk, list);
+        HIP_TRY(hipGetLastError());
+        uint32_t left = 0;
+        unsigned long long logged = 0;
+        HIP_TRY(hipMemcpyAsync(&left, &ctr->left, sizeof(left), hipMemcpyDeviceToHost, c->stream));
+        if (c->T.log_cap)
+          HIP_TRY(hipMemcpyAsync(&logged, c->T.log_n, sizeof(logged), hipMemcpyDeviceToHost,
+                                 c->stream));
+        HIP_TRY(hipStreamSynchronize(c->stream));
+        if (left > going) {
+          set_err("ssolh_solve: %u paths go on of %u", left, going);
           return SSOLH_ERR_LIMIT;
         }
-        const uint32_t k = launched & 1u;
-        hipError_t e = hipGraphLaunch(exec, c->stream);
-        if (e == hipSuccess)
-          e = hipMemcpyAsync(c->pinned + k, cnt, sizeof(unsigned), hipMemcpyDeviceToHost,
-                             c->stream);
-        if (e == hipSuccess) e = hipEventRecord(c->gev[k], c->stream);
-        if (e != hipSuccess) {
-          set_err("graph solve: %s", hipGetErrorString(e));
-          (void)hipStreamSynchronize(c->stream);
-          return -(int)e;
-        }
-        ++launched;
-        iter += gi;
-        wave_iter += gi;
+        going = left;
+        if (!going) break;
+        args.list = list;
+        // past half full, the log is summed before it overflows into atomics
+        if (logged && logged >= c->T.log_cap / 2) if ((r = log_flush())) return r;
       }
-      const uint32_t k = seen & 1u;
-      const hipError_t se = hipEventSynchronize(c->gev[k]);
-      if (se != hipSuccess) { set_err("graph solve: %s", hipGetErrorString(se)); return -(int)se; }
-      count = c->pinned[k];
-      ++seen;
-    }
-    const hipError_t se = hipStreamSynchronize(c->stream);
-    if (se != hipSuccess) { set_err("graph solve: %s", hipGetErrorString(se)); return -(int)se; }
-    return 0;
-  };
-
-  const uint64_t chunk = chunked ? slots : N;  // realisations started per wavefront
-  int gerr = 0;
-  uint32_t waves = 0;
-  for (uint64_t first = 0; first < N && !gerr; first += chunk) {
-    const uint32_t count = (uint32_t)std::min<uint64_t>(N - first, slots);
-    wave_iter = 0;
-    ++waves;
-    if ((gerr = start(first, count))) break;
-    if (!graph_iters) {
-      gerr = drain_host(count);
+      std::swap(from, to);
+      args.in = from;
+      args.out = to;
+      if ((r = resume(going))) return r;
+    } while (!run_through(going));
+    HIP_TRY(hipEventRecord(c->ev[2], c->stream));
+    if (c->T.log_cap) {
+      if ((r = log_flush())) return r;
     } else {
-      if (!exec) {
-        HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        int cr = 0;
-        for (uint32_t k = 0; k < gi && !cr; ++k) cr = iteration((int)(k & 1), max_blocks);
-        const hipError_t ce = hipStreamEndCapture(c->stream, &graph);
-        if (cr) { if (graph) (void)hipGraphDestroy(graph); return cr; }
-        HIP_TRY(ce);
-        const hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-        if (ie != hipSuccess) {
-          (void)hipGraphDestroy(graph);
-          HIP_TRY(ie);
-        }
-      }
-      gerr = drain_graph(count);
+      HIP_TRY(hipStreamSynchronize(c->stream));
     }
-    if (!gerr) gerr = log_flush();
-    if (!chunked || gerr) break;  // refill: one wavefront runs every realisation
-    // Too many failed paths: like the reference's loop, which skips every
-    // realisation not yet started once the limit is hit
-    // (src/ssol_solver.c:1227, 1241-1245), no further chunk starts. The
-    // stream is idle here (the drain synchronised it).
-    unsigned aborted = 0;
-    const hipError_t ae = hipMemcpy(&aborted, &ctr->aborted, sizeof(aborted), hipMemcpyDeviceToHost);
-    if (ae != hipSuccess) { set_err("ssolh_solve: %s", hipGetErrorString(ae)); gerr = -(int)ae; break; }
-    if (aborted) break;
+    float t = 0;
+    (void)hipEventElapsedTime(&t, c->ev[1], c->ev[2]);
+    ms_path += t;
   }
-  if (exec) (void)hipGraphExecDestroy(exec);
-  if (graph) (void)hipGraphDestroy(graph);
-  if (gerr) return gerr;
   // fold the stripes
   auto fold = [&](auto* base, size_t nn, uint32_t stripes) -> int {
     if (stripes > 1 && nn) {
@@ -3831,15 +2790,16 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
   HIP_TRY(hipStreamSynchronize(c->stream));
   (void)hipEventElapsedTime(&total_ms, c->ev[0], c->ev[3]);
   HIP_TRY(hipMemcpy(&c->last, c->counters.p, sizeof(Counters), hipMemcpyDeviceToHost));
-  c->segments = c->last.segments;
+  double rays = 0;  // counted beside job 0's global fields
+  HIP_TRY(hipMemcpy(&rays, c->T.global + 13, sizeof(rays), hipMemcpyDeviceToHost));
+  c->segments = (uint64_t)rays;
   if (trk) HIP_TRY(hipMemcpy(&c->trk_nvtx, c->trk_count.p, sizeof(c->trk_nvtx), hipMemcpyDeviceToHost));
   c->kernel_ms = total_ms;
-  c->trace_ms = ms_trace;
-  c->shade_ms = ms_shade;
-  c->iterations = iter;
-  c->wavefronts = waves;
-  c->refilled = slots < N && !chunked;
-  c->keys_clean = !arena;  // drained: every finished path cleared its keys
+  c->trace_ms = ms_path;  // tracing and shading are one kernel
+  c->shade_ms = 0;
+  c->iterations = c->last.iterations + c->last.gens;
+  c->wavefronts = c->last.wavefronts;
+  c->refilled = refill;
   return 0;
 }
 
@@ -3857,8 +2817,7 @@ SSOLH_API int ssolh_solve(ssolh_context* c, const struct ssolh_solve_args* a) {
   HIP_TRY(hipSetDevice(c->device));
   const uint32_t npend = a->pending_entries ? a->pending_entries : 4;
   return run_solve(c, a->realisations, a->max_failed, a->rng_key, a->rng_counter,
-                   a->precision == SSOLH_FP32, a->path_slots, npend, 1, nullptr, nullptr,
-                   a->graph_iterations);
+                   a->precision == SSOLH_FP32, a->path_slots, npend, 1, nullptr, nullptr);
 }
 
 SSOLH_API int ssolh_solve_noalloc(ssolh_context* c, const struct ssolh_solve_args* a,
@@ -3881,10 +2840,8 @@ SSOLH_API int ssolh_solve_noalloc(ssolh_context* c, const struct ssolh_solve_arg
   // The solve's buffers come from the scratch array: the context's own
   // buffers are set aside for the call (nothing is freed or allocated) and
   // put back after it.
-  DevBuf* bufs[] = {&c->state,        &c->rays,         &c->hits,        &c->lists[0],
-                    &c->lists[1],     &c->emitted,      &c->block_emits, &c->block_offsets,
-                    &c->scan_chunks,  &c->counters,     &c->tallies,     &c->start_sort,
-                    &c->trace_ovf};
+  DevBuf* bufs[] = {&c->start_sort, &c->queue[0], &c->queue[1], &c->list,
+                    &c->pend,       &c->counters, &c->tallies,  &c->trace_ovf};
   constexpr size_t NB = sizeof(bufs) / sizeof(bufs[0]);
   DevBuf saved[NB];
   for (size_t i = 0; i < NB; ++i) {
@@ -3894,7 +2851,7 @@ SSOLH_API int ssolh_solve_noalloc(ssolh_context* c, const struct ssolh_solve_arg
   Arena arena{(char*)c->scratch, SCRATCH_BYTES, 0};
   const uint32_t npend = a->pending_entries ? a->pending_entries : 4;
   int r = run_solve(c, a->realisations, a->max_failed, a->rng_key, a->rng_counter,
-                    a->precision == SSOLH_FP32, a->path_slots, npend, 1, nullptr, nullptr, 0,
+                    a->precision == SSOLH_FP32, a->path_slots, npend, 1, nullptr, nullptr,
                     nullptr, nullptr, &arena);
   if (!r) r = ssolh_tallies_download(c, out);
   for (size_t i = 0; i < NB; ++i) *bufs[i] = saved[i];
@@ -3922,7 +2879,7 @@ SSOLH_API int ssolh_solve_batch(ssolh_context* c, const struct ssolh_batch_args*
   std::vector<ssolh_sun> suns(a->suns, a->suns + a->nsuns);
   int r = run_solve(c, first[a->nsuns], a->max_failed, a->rng_key, a->rng_counter,
                     a->precision == SSOLH_FP32, a->path_slots, npend, njobs, first.data(),
-                    suns.data(), a->graph_iterations);
+                    suns.data());
   if (r) return r;
   std::vector<double> g((size_t)njobs * 16);
   HIP_TRY(hipMemcpy(g.data(), c->T.global, g.size() * sizeof(double), hipMemcpyDeviceToHost));
@@ -3956,7 +2913,7 @@ SSOLH_API int ssolh_solve_adjoint(ssolh_context* c, const struct ssolh_adjoint_a
   const uint32_t npend = a->solve.pending_entries ? a->solve.pending_entries : 4;
   int r = run_solve(c, a->solve.realisations, a->solve.max_failed, a->solve.rng_key,
                     a->solve.rng_counter, false, a->solve.path_slots, npend, 1, nullptr, nullptr,
-                    a->solve.graph_iterations, &h);
+                    &h);
   if (r) return r;
   HIP_TRY(hipMemcpy(grad, c->adj_grad.p, (size_t)a->nparams * 3 * sizeof(double),
                     hipMemcpyDeviceToHost));
@@ -3985,7 +2942,7 @@ SSOLH_API int ssolh_solve_tracked(ssolh_context* c, const struct ssolh_solve_arg
   TrackHost h{t->sun_ray_length, t->infinite_ray_length, t->max_vertices};
   const uint32_t npend = a->pending_entries ? a->pending_entries : 4;
   int r = run_solve(c, a->realisations, a->max_failed, a->rng_key, a->rng_counter, false,
-                    a->path_slots, npend, 1, nullptr, nullptr, 0, nullptr, &h);
+                    a->path_slots, npend, 1, nullptr, nullptr, nullptr, &h);
   if (r) return r;
   *nvertices = c->trk_nvtx;
   return 0;
