@@ -1486,14 +1486,75 @@ hipError_t start_sort_bytes(uint32_t count, uint32_t bits, hipStream_t stream, s
                                             (uint32_t*)nullptr, (int)count, 0, (int)bits, stream);
 }
 
-// Sum of the stripes of a striped tally into stripe 0
-template <typename T>
-__global__ void k_fold(T* base, size_t n, uint32_t stripes) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  T s = base[i];
-  for (uint32_t k = 1; k < stripes; ++k) s += base[(size_t)k * n + i];
-  base[i] = s;
+// Sums of the stripes of every tally, in one launch, and the solve's
+// counters beside them. A block takes a tile of 1024 / rows consecutive
+// elements of one tally, its rows each every rows-th stripe, and adds the rows
+// up in LDS: a tally of 40 elements in 256 stripes (one receiver) takes 16
+// loads in a row instead of 256, and the launch as long as the largest tally
+// takes to read (field of 100 paraboloids, 36 MB of stripes: six launches of
+// together 507 us, one thread per element -> one of 25 us).
+constexpr int FOLD_THREADS = 1024, FOLD_ROWS = 16;
+struct FoldPart {
+  const void* src;     // [stripes][n], doubles or (whole) 64-bit counts
+  void* dst;           // [n], may be stripe 0 of src
+  uint64_t n;
+  uint32_t stripes;    // a power of two
+  uint32_t first;      // first block of the part
+  uint32_t whole;
+};
+constexpr int FOLD_PARTS = 6;
+struct FoldArgs {
+  FoldPart part[FOLD_PARTS];
+  const Counters* C;
+  Counters* C_out;
+};
+
+// Adds v to the sum s + e; e collects the rounding errors of s (Knuth's
+// two-sum), so the fold adds none of its own to a tally: variances come from
+// the difference of two of them
+__device__ __forceinline__ void add_to(double& s, double& e, double v) {
+  const double t = s + v, b = t - s;
+  e += (s - (t - b)) + (v - b);
+  s = t;
+}
+
+__device__ __forceinline__ void fold_tile(const FoldPart& p, uint64_t tile, double* lds) {
+  const uint32_t rows = min(p.stripes, (uint32_t)FOLD_ROWS), cols = FOLD_THREADS / rows;
+  const uint32_t row = threadIdx.x / cols, col = threadIdx.x % cols;
+  const uint64_t i = tile * cols + col;
+  double s = 0, e = 0;
+  if (i < p.n)
+    for (uint32_t k = row; k < p.stripes; k += rows) add_to(s, e, ((const double*)p.src)[k * p.n + i]);
+  lds[threadIdx.x] = s;
+  lds[FOLD_THREADS + threadIdx.x] = e;
+  __syncthreads();
+  if (row == 0 && i < p.n) {
+    for (uint32_t k = 1; k < rows; ++k) {
+      add_to(s, e, lds[k * cols + col]);
+      e += lds[FOLD_THREADS + k * cols + col];
+    }
+    ((double*)p.dst)[i] = s + e;
+  }
+}
+
+// The same for counts, which few tallies have: one thread per element
+__device__ __forceinline__ void fold_counts(const FoldPart& p, uint64_t tile) {
+  const uint64_t i = tile * FOLD_THREADS + threadIdx.x;
+  if (i >= p.n) return;
+  unsigned long long s = 0;
+#pragma unroll 8
+  for (uint32_t k = 0; k < p.stripes; ++k) s += ((const unsigned long long*)p.src)[k * p.n + i];
+  ((unsigned long long*)p.dst)[i] = s;
+}
+
+__global__ void __launch_bounds__(FOLD_THREADS) k_fold(FoldArgs a) {
+  __shared__ double lds[2 * FOLD_THREADS];
+  if (blockIdx.x == 0 && threadIdx.x == 0) *a.C_out = *a.C;
+  int k = FOLD_PARTS - 1;
+  while (k > 0 && blockIdx.x < a.part[k].first) --k;
+  const FoldPart& p = a.part[k];
+  if (p.whole) fold_counts(p, blockIdx.x - p.first);
+  else fold_tile(p, blockIdx.x - p.first, lds);
 }
 
 // -------------------------------------------------------------------------
@@ -1584,6 +1645,8 @@ struct DevBuf {
 // copy is reached through the pointer hipGetSymbolAddress returns with that
 // device current (kept per device by ssolh_create).
 constexpr size_t SCRATCH_BYTES = size_t(64) << 20;
+// folded tallies of up to so many bytes are kept in pinned host memory
+constexpr size_t STAGE_MAX = size_t(64) << 20;
 // records of the per-primitive log (84 B each plus 12 B of sort arrays)
 constexpr uint64_t LOG_MAX_RECORDS = uint64_t(1) << 27;
 static __device__ __align__(256) unsigned char scratch[SCRATCH_BYTES];
@@ -1649,7 +1712,14 @@ struct ssolh_context {
   uint32_t njobs = 1;
   const ShapeQ* shapeq = nullptr;  // per shape, in scene_bufs
   Tallies T{};
-  size_t tally_bytes = 0;
+  // folded tallies: counters, then the tallies one after the other, copied to
+  // `stage` (pinned) by each solve when they take at most STAGE_MAX bytes;
+  // F: where the folded tallies are on the device
+  DevBuf folded;
+  Tallies F{};
+  void* stage = nullptr;
+  size_t stage_bytes = 0;
+  bool staged = false;
   // last solve
   Counters last{};
   uint64_t segments = 0;
@@ -1925,11 +1995,12 @@ SSOLH_API int ssolh_destroy(ssolh_context* c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   free_scene(c);
   for (DevBuf* b : {&c->start_sort, &c->queue[0], &c->queue[1], &c->list, &c->pend, &c->counters,
-                    &c->tallies, &c->jobs, &c->trace_ovf, &c->lbvh, &c->render, &c->plog,
+                    &c->tallies, &c->folded, &c->jobs, &c->trace_ovf, &c->lbvh, &c->render, &c->plog,
                     &c->adj_state, &c->adj_in, &c->adj_grad, &c->trk_vtx, &c->trk_type,
                     &c->trk_seq, &c->trk_count, &c->trk_pos})
     if (b->p) (void)hipFree(b->p);
   for (auto& e : c->ev) if (e) (void)hipEventDestroy(e);
+  if (c->stage) (void)hipHostFree(c->stage);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
   return 0;
@@ -2550,7 +2621,6 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
 
   // tallies (striped where many waves meet, see Tallies)
   if ((r = alloc(c->tallies, tally_bytes))) return r;
-  c->tally_bytes = tally_bytes;
   double* tb = (double*)c->tallies.p;
   c->T.global = tb;
   c->T.rcv = c->T.global + n_global;
@@ -2771,27 +2841,68 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
     (void)hipEventElapsedTime(&t, c->ev[1], c->ev[2]);
     ms_path += t;
   }
-  // fold the stripes
-  auto fold = [&](auto* base, size_t nn, uint32_t stripes) -> int {
-    if (stripes > 1 && nn) {
-      k_fold<<<(unsigned)((nn + 255) / 256), 256, 0, c->stream>>>(base, nn, stripes);
-      HIP_TRY(hipGetLastError());
+  // fold the stripes: into one buffer, copied whole to pinned host memory;
+  // from the scratch array, in place
+  const size_t parts[FOLD_PARTS] = {(size_t)njobs * 16, (size_t)c->nrcv * 40, (size_t)c->nsamp * 4,
+                                    (size_t)c->nsamp * c->nrcv * 40, (size_t)c->nprim * 40,
+                                    (size_t)c->nsamp};
+  const uint32_t stripes[FOLD_PARTS] = {sg, sr, ss, sx, sp, ss};
+  void* const src[FOLD_PARTS] = {c->T.global, c->T.rcv, c->T.samp, c->T.sxr, c->T.prim,
+                                 c->T.samp_count};
+  constexpr size_t head = (sizeof(Counters) + 63) / 64 * 64;
+  size_t folded = head;
+  for (size_t x : parts) folded += x * 8;
+  FoldArgs fold{};
+  fold.C = fold.C_out = ctr;
+  c->F = c->T;
+  c->staged = false;
+  if (!arena) {
+    if ((r = alloc(c->folded, folded))) return r;
+    if (folded <= STAGE_MAX && c->stage_bytes < folded) {
+      if (c->stage) (void)hipHostFree(c->stage);
+      c->stage = nullptr;
+      c->stage_bytes = 0;
+      if (hipHostMalloc(&c->stage, folded, hipHostMallocDefault) == hipSuccess)
+        c->stage_bytes = folded;
+      else
+        (void)hipGetLastError();  // then read from the device
     }
-    return 0;
-  };
-  if ((r = fold(c->T.global, (size_t)njobs * 16, sg))) return r;
-  if ((r = fold(c->T.rcv, (size_t)c->nrcv * 40, sr))) return r;
-  if ((r = fold(c->T.samp, (size_t)c->nsamp * 4, ss))) return r;
-  if ((r = fold(c->T.samp_count, (size_t)c->nsamp, ss))) return r;
-  if ((r = fold(c->T.sxr, (size_t)c->nsamp * c->nrcv * 40, sx))) return r;
-  if ((r = fold(c->T.prim, (size_t)c->nprim * 40, sp))) return r;
+    c->staged = c->stage_bytes >= folded;
+    fold.C_out = (Counters*)c->folded.p;
+    double* d = (double*)((char*)c->folded.p + head);
+    c->F.global = d; d += parts[0];
+    c->F.rcv = d; d += parts[1];
+    c->F.samp = d; d += parts[2];
+    c->F.sxr = d; d += parts[3];
+    c->F.prim = d; d += parts[4];
+    c->F.samp_count = (unsigned long long*)d;
+  }
+  void* const dst[FOLD_PARTS] = {c->F.global, c->F.rcv, c->F.samp, c->F.sxr, c->F.prim,
+                                 c->F.samp_count};
+  uint32_t blocks = 0;
+  for (int k = 0; k < FOLD_PARTS; ++k) {
+    const bool whole = k == FOLD_PARTS - 1;
+    const uint32_t cols = whole ? FOLD_THREADS
+                                : FOLD_THREADS / std::min<uint32_t>(stripes[k], FOLD_ROWS);
+    fold.part[k] = FoldPart{src[k], dst[k], parts[k], stripes[k], blocks, whole};
+    blocks += (uint32_t)((parts[k] + cols - 1) / cols);
+  }
+  k_fold<<<blocks, FOLD_THREADS, 0, c->stream>>>(fold);
+  HIP_TRY(hipGetLastError());
+  if (c->staged)
+    HIP_TRY(hipMemcpyAsync(c->stage, c->folded.p, folded, hipMemcpyDeviceToHost, c->stream));
   float total_ms = 0;
   HIP_TRY(hipEventRecord(c->ev[3], c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
   (void)hipEventElapsedTime(&total_ms, c->ev[0], c->ev[3]);
-  HIP_TRY(hipMemcpy(&c->last, c->counters.p, sizeof(Counters), hipMemcpyDeviceToHost));
   double rays = 0;  // counted beside job 0's global fields
-  HIP_TRY(hipMemcpy(&rays, c->T.global + 13, sizeof(rays), hipMemcpyDeviceToHost));
+  if (c->staged) {
+    memcpy(&c->last, c->stage, sizeof(Counters));
+    memcpy(&rays, (char*)c->stage + head + 13 * 8, sizeof(rays));
+  } else {
+    HIP_TRY(hipMemcpy(&c->last, fold.C_out, sizeof(Counters), hipMemcpyDeviceToHost));
+    HIP_TRY(hipMemcpy(&rays, c->F.global + 13, sizeof(rays), hipMemcpyDeviceToHost));
+  }
   c->segments = (uint64_t)rays;
   if (trk) HIP_TRY(hipMemcpy(&c->trk_nvtx, c->trk_count.p, sizeof(c->trk_nvtx), hipMemcpyDeviceToHost));
   c->kernel_ms = total_ms;
@@ -2806,6 +2917,17 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
 }  // namespace
 
 extern "C" {
+
+// `bytes` of the folded tallies at device address `src` (in c->F)
+static int tallies_to(const ssolh_context* c, void* dst, const void* src, size_t bytes) {
+  if (!bytes) return 0;
+  if (c->staged) {
+    memcpy(dst, (const char*)c->stage + ((const char*)src - (const char*)c->folded.p), bytes);
+    return 0;
+  }
+  HIP_TRY(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
+  return 0;
+}
 
 SSOLH_API int ssolh_solve(ssolh_context* c, const struct ssolh_solve_args* a) {
   if (!c || !a || !a->realisations) { set_err("ssolh_solve: invalid arguments"); return SSOLH_ERR_ARG; }
@@ -2882,7 +3004,7 @@ SSOLH_API int ssolh_solve_batch(ssolh_context* c, const struct ssolh_batch_args*
                     suns.data());
   if (r) return r;
   std::vector<double> g((size_t)njobs * 16);
-  HIP_TRY(hipMemcpy(g.data(), c->T.global, g.size() * sizeof(double), hipMemcpyDeviceToHost));
+  if ((r = tallies_to(c, g.data(), c->F.global, g.size() * sizeof(double)))) return r;
   for (uint32_t j = 0; j < njobs; ++j) {
     memcpy(out[j].global, &g[(size_t)j * 16], 12 * sizeof(double));
     out[j].realisation_count = (uint64_t)g[(size_t)j * 16 + 12];
@@ -2918,7 +3040,7 @@ SSOLH_API int ssolh_solve_adjoint(ssolh_context* c, const struct ssolh_adjoint_a
   HIP_TRY(hipMemcpy(grad, c->adj_grad.p, (size_t)a->nparams * 3 * sizeof(double),
                     hipMemcpyDeviceToHost));
   double n = 0;
-  HIP_TRY(hipMemcpy(&n, c->T.global + 12, sizeof(double), hipMemcpyDeviceToHost));
+  if ((r = tallies_to(c, &n, c->F.global + 12, sizeof(double)))) return r;
   for (size_t i = 0; i < (size_t)a->nparams * 3; ++i) grad[i] = n > 0 ? grad[i] / n : 0.0;
   return 0;
 }
@@ -2973,16 +3095,15 @@ SSOLH_API int ssolh_tallies_download(ssolh_context* c, struct ssolh_tallies* o) 
   HIP_TRY(hipSetDevice(c->device));
   const size_t n_rcv = (size_t)c->nrcv * 40, n_samp = (size_t)c->nsamp * 4;
   const size_t n_sxr = (size_t)c->nsamp * c->nrcv * 40, n_prim = (size_t)c->nprim * 40;
-  HIP_TRY(hipMemcpy(o->global, c->T.global, 12 * sizeof(double), hipMemcpyDeviceToHost));
-  if (o->receivers && n_rcv) HIP_TRY(hipMemcpy(o->receivers, c->T.rcv, n_rcv * 8, hipMemcpyDeviceToHost));
-  if (o->sampled && n_samp) HIP_TRY(hipMemcpy(o->sampled, c->T.samp, n_samp * 8, hipMemcpyDeviceToHost));
-  if (o->sampled_count && c->nsamp)
-    HIP_TRY(hipMemcpy(o->sampled_count, c->T.samp_count, c->nsamp * 8, hipMemcpyDeviceToHost));
-  if (o->sampled_x_receivers && n_sxr)
-    HIP_TRY(hipMemcpy(o->sampled_x_receivers, c->T.sxr, n_sxr * 8, hipMemcpyDeviceToHost));
-  if (o->primitives && n_prim) HIP_TRY(hipMemcpy(o->primitives, c->T.prim, n_prim * 8, hipMemcpyDeviceToHost));
   double cnt0 = 0;
-  HIP_TRY(hipMemcpy(&cnt0, c->T.global + 12, sizeof(double), hipMemcpyDeviceToHost));
+  int r = tallies_to(c, o->global, c->F.global, 12 * sizeof(double));
+  if (!r) r = tallies_to(c, &cnt0, c->F.global + 12, sizeof(double));
+  if (!r && o->receivers) r = tallies_to(c, o->receivers, c->F.rcv, n_rcv * 8);
+  if (!r && o->sampled) r = tallies_to(c, o->sampled, c->F.samp, n_samp * 8);
+  if (!r && o->sampled_count) r = tallies_to(c, o->sampled_count, c->F.samp_count, c->nsamp * 8);
+  if (!r && o->sampled_x_receivers) r = tallies_to(c, o->sampled_x_receivers, c->F.sxr, n_sxr * 8);
+  if (!r && o->primitives) r = tallies_to(c, o->primitives, c->F.prim, n_prim * 8);
+  if (r) return r;
   o->realisation_count = (uint64_t)cnt0;
   o->failed_count = c->last.failed;
   o->segments = c->segments;
