@@ -204,12 +204,12 @@ struct Counters {
 struct Tallies {
   double* global;   // [mask_g+1][njobs][16]: 6 fields x {w, w2}, then the
                     // realisation count (exact below 2^53); one 128-byte line
-  double* rcv;      // [mask_r+1][nrcv][2][10][2]
+  double* rcv;      // [nrcv][2][10][2]: zero until folded (k_fold_rcv)
   double* samp;     // [mask_s+1][nsamp][2][2]
   unsigned long long* samp_count;    // [mask_s+1][nsamp]
   double* sxr;      // [mask_x+1][nsamp][nrcv][2][10][2]
   double* prim;     // [mask_p+1][nprim][2][10][2]
-  uint32_t mask_g, mask_r, mask_s, mask_x, mask_p;
+  uint32_t mask_g, mask_s, mask_x, mask_p;
   uint32_t nrcv, nsamp, njobs;
   uint64_t nprim;
   // Log of finished paths' per-primitive entries (prim_add), reduced into
@@ -308,23 +308,46 @@ __device__ __forceinline__ double dpp_move(double v) {
   return __longlong_as_double((long long)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo));
 }
 
-__device__ __forceinline__ double read_lane(double v, int lane) {
-  const uint64_t b = (uint64_t)__double_as_longlong(v);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), lane);
-  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
-
-// Sum over the 64 lanes of a wave; every lane must be active. DPP moves
-// sum within quads (quad_perm [1,0,3,2], [2,3,0,1]), half rows
-// (row_half_mirror) and rows of 16 (row_mirror); the four row sums are
-// then read from lanes 0, 16, 32, 48.
-__device__ __forceinline__ double wave_sum(double v) {
-  v += dpp_move<0xB1>(v);
-  v += dpp_move<0x4E>(v);
-  v += dpp_move<0x141>(v);
-  v += dpp_move<0x140>(v);
-  return (read_lane(v, 0) + read_lane(v, 16)) + (read_lane(v, 32) + read_lane(v, 48));
+// Sums of N values (a multiple of 4) over the 64 lanes of a wave, every lane
+// active: lane l returns the total of value (l / 16) * N / 4 + l % 16, where
+// l % 16 < N / 4. Two swaps halve the values in hand instead of adding both
+// halves of each: v_permlane32_swap leaves value i in the lower and value i +
+// N/2 in the upper 32 lanes, v_permlane16_swap does the same for rows of 16;
+// DPP moves then add up the row within quads (quad_perm [1,0,3,2], [2,3,0,1]),
+// half rows (row_half_mirror) and the row (row_mirror). 20 values: 105
+// instructions, where summing each over all lanes takes 540.
+template <int N>
+__device__ __forceinline__ double wave_totals(const double (&v)[N]) {
+  static_assert(N % 4 == 0 && N / 4 <= 16, "values per row");
+  auto swapped = [](double a, double b, auto swap) {
+    const uint64_t x = (uint64_t)__double_as_longlong(a), y = (uint64_t)__double_as_longlong(b);
+    const auto lo = swap((uint32_t)x, (uint32_t)y);
+    const auto hi = swap((uint32_t)(x >> 32), (uint32_t)(y >> 32));
+    return __longlong_as_double((long long)(((uint64_t)hi[0] << 32) | lo[0])) +
+           __longlong_as_double((long long)(((uint64_t)hi[1] << 32) | lo[1]));
+  };
+  double h[N / 2], r[N / 4];
+#pragma unroll
+  for (int i = 0; i < N / 2; ++i)
+    h[i] = swapped(v[i], v[i + N / 2], [](uint32_t x, uint32_t y) {
+      return __builtin_amdgcn_permlane32_swap(x, y, false, false);
+    });
+#pragma unroll
+  for (int i = 0; i < N / 4; ++i)
+    r[i] = swapped(h[i], h[i + N / 4], [](uint32_t x, uint32_t y) {
+      return __builtin_amdgcn_permlane16_swap(x, y, false, false);
+    });
+#pragma unroll
+  for (int i = 0; i < N / 4; ++i) {
+    r[i] += dpp_move<0xB1>(r[i]);
+    r[i] += dpp_move<0x4E>(r[i]);
+    r[i] += dpp_move<0x141>(r[i]);
+    r[i] += dpp_move<0x140>(r[i]);
+  }
+  double s = r[0];
+#pragma unroll
+  for (int i = 1; i < N / 4; ++i) s = (__lane_id() & 15u) == (unsigned)i ? r[i] : s;
+  return s;
 }
 
 __device__ __forceinline__ unsigned lane_id() { return __lane_id(); }
@@ -333,30 +356,40 @@ __device__ __forceinline__ void atomic_add(double* p, double v) {
   if (v != 0) unsafeAtomicAdd(p, v);
 }
 
-// Adds the NV values of each participating lane at base[key*NV + i]. Lanes
-// sharing the first participant's key are reduced across the wave and
-// flushed by one lane; the others use per-lane atomics. Must be called by
-// the whole wave.
-template <int NV, int STRIDE = NV>
-__device__ void keyed_add(bool has, uint64_t key, const double* v, double* base) {
-  const uint64_t mask = __ballot(has);
-  if (!mask) return;
-  const int leader = __ffsll((unsigned long long)mask) - 1;
-  const uint64_t lkey = __shfl(key, leader, 64);
-  const bool match = has && key == lkey;
-  if (__popcll(__ballot(match)) > 1) {
-    // several lanes share the key: one reduction, one set of atomics
+// Adds the wave's totals of v to base[i], i < NV, each by one lane. Every lane
+// of the wave calls it.
+template <int NV, int N>
+__device__ __forceinline__ void add_totals(const double (&v)[N], double* base) {
+  const double s = wave_totals<N>(v);
+  const unsigned j = lane_id() & 15u, i = (lane_id() >> 4) * (N / 4) + j;
+  if (j < N / 4 && i < NV) atomic_add(base + i, s);
+}
+
+// Adds the NV values of each participating lane at base[key*STRIDE + i]. The
+// lanes of each key that several lanes hold are reduced across the wave and
+// added by one atomic per value; a lane with a key of its own adds for
+// itself. FP64 atomics issue at one rate for the whole device (about 88 of 20
+// values per microsecond and CU), so a reduction pays from two lanes on.
+// v is padded to N values, a multiple of 4. Must be called by the whole wave.
+template <int NV, int STRIDE = NV, int N>
+__device__ __forceinline__ void keyed_add(bool has, uint64_t key, const double (&v)[N],
+                                          double* base) {
+  bool todo = has, alone = false;
+  for (uint64_t mask = __ballot(todo); mask; mask = __ballot(todo)) {
+    const int leader = __ffsll((unsigned long long)mask) - 1;
+    const uint64_t lkey = __shfl(key, leader, 64);
+    const bool match = todo && key == lkey;
+    if (__popcll(__ballot(match)) > 1) {
+      double m[N];
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const double s = wave_sum(match ? v[i] : 0.0);
-      if ((int)lane_id() == leader) atomic_add(base + lkey * STRIDE + i, s);
+      for (int i = 0; i < N; ++i) m[i] = match ? v[i] : 0.0;
+      add_totals<NV, N>(m, base + lkey * STRIDE);
+    } else {
+      alone = alone || match;
     }
-    if (has && !match) {
-#pragma unroll
-      for (int i = 0; i < NV; ++i) atomic_add(base + key * STRIDE + i, v[i]);
-    }
-  } else if (has) {
-    // keys all distinct so far: per-lane atomics, no reduction
+    todo = todo && !match;
+  }
+  if (alone) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) atomic_add(base + key * STRIDE + i, v[i]);
   }
@@ -410,15 +443,6 @@ __device__ void prim_add(const Tallies& T, bool has, uint32_t key, const R* a, d
 // keys so.
 constexpr uint32_t PRIM_ROUNDS = 8;
 
-__device__ __forceinline__ void prim_flush_run(double* pb, uint32_t key, const double* acc,
-                                               int leader) {
-#pragma unroll
-  for (int f = 0; f < 20; ++f) {
-    const double s = wave_sum(acc[f]);
-    if ((int)lane_id() == leader) atomic_add(pb + (size_t)key * 20u + f, s);
-  }
-}
-
 __global__ void __launch_bounds__(256) k_prim_reduce(const uint32_t* __restrict__ skey,
                                                      const uint32_t* __restrict__ sidx,
                                                      const double* __restrict__ val, uint32_t m,
@@ -452,7 +476,7 @@ __global__ void __launch_bounds__(256) k_prim_reduce(const uint32_t* __restrict_
     const uint32_t k0 = __shfl(key, 0, 64);
     const bool one_key = __ballot(in && key == k0) == inmask;
     if (!(one_key && k0 == acc_key) && acc_key != NONE) {
-      prim_flush_run(pb, acc_key, acc, 0);
+      add_totals<20>(acc, pb + (size_t)acc_key * 20u);
 #pragma unroll
       for (int f = 0; f < 20; ++f) acc[f] = 0.0;
       acc_key = NONE;
@@ -478,11 +502,11 @@ __global__ void __launch_bounds__(256) k_prim_reduce(const uint32_t* __restrict_
         run[2 * f] = match ? x[f] : 0.0;
         run[2 * f + 1] = match ? x[f] * x[f] : 0.0;
       }
-      prim_flush_run(pb, lkey, run, leader);
+      add_totals<20>(run, pb + (size_t)lkey * 20u);
       todo = todo && !match;
     }
   }
-  if (acc_key != NONE) prim_flush_run(pb, acc_key, acc, 0);
+  if (acc_key != NONE) add_totals<20>(acc, pb + (size_t)acc_key * 20u);
 }
 
 __global__ void k_iota32(uint32_t* a, uint32_t n) {
@@ -1547,6 +1571,30 @@ __device__ __forceinline__ void fold_counts(const FoldPart& p, uint64_t tile) {
   ((unsigned long long*)p.dst)[i] = s;
 }
 
+// The receiver tally: a realisation starts on one sampled instance, so it is
+// the folded sampled x receiver tally summed over the instances. n: doubles
+// per instance, gridDim.y shares of the instances; rcv is zero before.
+__global__ void __launch_bounds__(FOLD_THREADS)
+k_fold_rcv(const double* __restrict__ sxr, uint64_t n, uint32_t nsamp, double* rcv) {
+  __shared__ double lds[2 * FOLD_THREADS];
+  constexpr uint32_t cols = FOLD_THREADS / FOLD_ROWS;
+  const uint32_t row = threadIdx.x / cols, col = threadIdx.x % cols;
+  const uint64_t i = (uint64_t)blockIdx.x * cols + col;
+  double s = 0, e = 0;
+  if (i < n)
+    for (uint32_t k = blockIdx.y * FOLD_ROWS + row; k < nsamp; k += gridDim.y * FOLD_ROWS)
+      add_to(s, e, sxr[k * n + i]);
+  lds[threadIdx.x] = s;
+  lds[FOLD_THREADS + threadIdx.x] = e;
+  __syncthreads();
+  if (row || i >= n) return;
+  for (uint32_t k = 1; k < FOLD_ROWS; ++k) {
+    add_to(s, e, lds[k * cols + col]);
+    e += lds[FOLD_THREADS + k * cols + col];
+  }
+  atomic_add(rcv + i, s + e);
+}
+
 __global__ void __launch_bounds__(FOLD_THREADS) k_fold(FoldArgs a) {
   __shared__ double lds[2 * FOLD_THREADS];
   if (blockIdx.x == 0 && threadIdx.x == 0) *a.C_out = *a.C;
@@ -1576,9 +1624,12 @@ __global__ void k_test_quadric(int quadric, double4 qp, uint32_t n, const double
   }
 }
 
-// One wave_sum per wave of 64 inputs (blocks of 64 threads: every lane active)
+// wave_totals of four copies of a wave's 64 inputs: each row of 16 lanes
+// returns the total of one (blocks of 64 threads: every lane active)
 __global__ void __launch_bounds__(64) k_test_wave_sum(const double* in, double* out) {
-  const double s = wave_sum(in[blockIdx.x * 64 + threadIdx.x]);
+  const double x = in[blockIdx.x * 64 + threadIdx.x];
+  const double v[4] = {x, x, x, x};
+  const double s = __shfl(wave_totals<4>(v), (int)(threadIdx.x & 48u), 64);
   out[blockIdx.x * 64 + threadIdx.x] = s;
 }
 
@@ -2435,7 +2486,7 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
       return (uint32_t)k;
     };
     sg = pow2_stripes((size_t)njobs * 16);
-    sr = pow2_stripes((size_t)c->nrcv * 40);
+    sr = 1;  // zeros: the fold sums it from the sampled x receiver tally
     ss = pow2_stripes((size_t)c->nsamp * 5);
     sx = pow2_stripes((size_t)c->nsamp * c->nrcv * 40);
     sp = pow2_stripes((size_t)c->nprim * 40);
@@ -2629,7 +2680,6 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
   c->T.prim = c->T.sxr + n_sxr;
   c->T.samp_count = (unsigned long long*)(c->T.prim + n_prim);
   c->T.mask_g = sg - 1;
-  c->T.mask_r = sr - 1;
   c->T.mask_s = ss - 1;
   c->T.mask_x = sx - 1;
   c->T.mask_p = sp - 1;
@@ -2889,6 +2939,12 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
   }
   k_fold<<<blocks, FOLD_THREADS, 0, c->stream>>>(fold);
   HIP_TRY(hipGetLastError());
+  if (c->nrcv && c->nsamp) {
+    const dim3 grid((unsigned)((parts[1] + FOLD_THREADS / FOLD_ROWS - 1) / (FOLD_THREADS / FOLD_ROWS)),
+                    std::min<uint32_t>((c->nsamp + 255) / 256, 64));
+    k_fold_rcv<<<grid, FOLD_THREADS, 0, c->stream>>>(c->F.sxr, parts[1], c->nsamp, c->F.rcv);
+    HIP_TRY(hipGetLastError());
+  }
   if (c->staged)
     HIP_TRY(hipMemcpyAsync(c->stage, c->folded.p, folded, hipMemcpyDeviceToHost, c->stream));
   float total_ms = 0;

@@ -534,7 +534,6 @@ __device__ __forceinline__ bool shade_path(const PathArgs& a, Path<F>& p,
           receiver_weights(in0, in1, in2, kabs, w10);
           if (!pend_add(a.W.pkey + p.slot, (real*)a.W.pval + p.slot, stride, a.W.npend, p.npk, rkey,
                         w10)) {
-            spill(T.rcv + (size_t)(blockIdx.x & T.mask_r) * T.nrcv * 40u, rkey, w10, &a.C->spills);
             spill(T.sxr + (size_t)(blockIdx.x & T.mask_x) * T.nsamp * T.nrcv * 40u,
                   (uint64_t)p.samp * S.nrcv * 2u + rkey, w10, &a.C->spills);
           }
@@ -616,13 +615,14 @@ __device__ __forceinline__ void flush_paths(const PathArgs& a, const Path<F>& p)
     const bool counted = done || p.fin == FIN_KILLED;
     const double g[6] = {p.cosf, p.pd[0], last ? real(0) : p.pv[1], last ? real(0) : p.pv[0],
                          p.pd[1], p.pd[2]};
-    double g2[13];
+    double g2[16];
     for (int i = 0; i < 6; ++i) {
       const double x = done ? g[i] * factor : 0.0;
       g2[2 * i] = x;
       g2[2 * i + 1] = x * x;
     }
     g2[12] = 1.0;
+    g2[13] = g2[14] = g2[15] = 0.0;
     keyed_add<13, 16>(counted, counted ? p.job : 0, g2,
                       T.global + (size_t)(blockIdx.x & T.mask_g) * T.njobs * 16u);
     const double s4[4] = {g2[0], g2[1], g2[4], g2[5]};
@@ -631,12 +631,12 @@ __device__ __forceinline__ void flush_paths(const PathArgs& a, const Path<F>& p)
     const unsigned long long nf = wave_count_add(p.fin == FIN_FAILED, &a.C->failed);
     if (p.fin == FIN_FAILED && nf + 1 >= a.prm.max_failed) atomicExch(&a.C->aborted, 1u);
   }
-  // Receiver entries, then per-primitive ones: the pending entries in turn,
+  // Receiver entries (sampled x receiver: the receiver tally is their sum,
+  // k_fold_rcv), then per-primitive ones: the pending entries in turn,
   // then the last hit, which joins the pending entry of its key (before
   // squaring) if the path holds one
   real dw[10];
   receiver_weights(p.pv[0], p.pv[1], p.pv[2], p.pv[3], dw);
-  double* rcv_base = T.rcv + (size_t)(blockIdx.x & T.mask_r) * T.nrcv * 40u;
   double* sxr_base = T.sxr + (size_t)(blockIdx.x & T.mask_x) * T.nsamp * T.nrcv * 40u;
   for (int which = 0; which < 2; ++which) {
     const uint32_t n = !done ? 0u : which ? p.nqk : p.npk;
@@ -670,7 +670,6 @@ __device__ __forceinline__ void flush_paths(const PathArgs& a, const Path<F>& p)
         v[2 * f] = x;
         v[2 * f + 1] = x * x;
       }
-      keyed_add<20>(has, has ? key : 0, v, rcv_base);
       keyed_add<20>(has, has ? (uint64_t)p.samp * (uint64_t)a.S.nrcv * 2u + key : 0, v, sxr_base);
     }
   }
@@ -679,7 +678,7 @@ __device__ __forceinline__ void flush_paths(const PathArgs& a, const Path<F>& p)
   if (ADJ) {
     const uint32_t pp = done ? a.A.p[p.slot] : NONE;
     const bool has = pp != NONE;
-    double v[3] = {0.0, 0.0, 0.0};
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
     if (has) {
       const double4 sc = a.A.s[p.slot];
       const double q = sc.w * factor;

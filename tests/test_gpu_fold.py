@@ -4,7 +4,8 @@ stripes into one buffer; ssolh_solve_noalloc folds them in place and, in its
 realisations, so the folded tallies agree up to the order of the FP64
 additions, at sizes on both sides of the kernel's tiles (1024 / min(16,
 stripes) elements): receivers of 2 to 2,178 triangles, 1 to 130 sampled
-instances. Order of additions: sums of at most n = 60,000 terms of one sign
+instances (300: several shares of the instances in k_fold_rcv, which sums the
+receiver tally from the sampled x receiver one). Order of additions: sums of at most n = 60,000 terms of one sign
 in two orders differ by at most 2 n 2^-53 = 1.3e-11 relative; counts are
 equal."""
 import ctypes as C
@@ -21,7 +22,8 @@ pytestmark = pytest.mark.gpu
 REALISATIONS = 60_000
 
 
-@pytest.mark.parametrize("heliostats,cells", [(1, 1), (2, 7), (25, 8), (63, 33), (130, 9)])
+@pytest.mark.parametrize("heliostats,cells", [(1, 1), (2, 7), (25, 8), (63, 33), (130, 9),
+                                              (300, 4)])
 def test_fold_into_buffer_matches_fold_in_place(gpu, heliostats, cells):
     spec = S.config2(0, n_helio=heliostats, radius=40.0 + 20.0 * heliostats ** 0.5, rcv_size=8.0,
                      rcv_cells=cells)
@@ -37,6 +39,10 @@ def test_fold_into_buffer_matches_fold_in_place(gpu, heliostats, cells):
     assert ref.t.segments > REALISATIONS
     assert ref.rcv.any() and ref.samp.any() and ref.prim.any()
     N._same(got, ref, 1.3e-11)
+    for o in (ref, got):
+        per_instance = o.sxr[:heliostats * 40].reshape(heliostats, 40)
+        assert np.count_nonzero(per_instance[:, 0]) == heliostats
+        assert np.allclose(o.rcv[:40], per_instance.sum(axis=0), rtol=1e-13, atol=0)
     lib.close()
 
 
