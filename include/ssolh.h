@@ -496,6 +496,13 @@ SSOLH_API int ssolh_test_threefry
 SSOLH_API int ssolh_test_wave_sum
   (ssolh_context* ctx, uint32_t nwaves, const double* in, double* out);
 
+/* Grouping of n items by key (start order, per-primitive log): order takes
+ * the item indices, those of key k at offsets[k] .. offsets[k + 1] - 1.
+ * key[i] < nkeys <= 16384 */
+SSOLH_API int ssolh_test_group
+  (ssolh_context* ctx, uint32_t n, uint32_t nkeys, const uint32_t* key, uint32_t* order,
+   uint32_t* offsets);
+
 /* Traversal stack of the renderer's trace kernel: caps the entries each lane
  * keeps in LDS (16, 24 or 32; 0 restores the default, the smallest that holds
  * the scene's bound) for the calls that follow, so that the rest of the bound

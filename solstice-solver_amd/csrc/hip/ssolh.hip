@@ -194,6 +194,9 @@ struct Counters {
   unsigned int wavefronts;          // wavefronts begun
   unsigned int iterations, gens;    // generations of rays: of the passes so far, of this one
   unsigned int left;                // length of the list of paths that go on
+  unsigned int log_flushes;         // reductions of the per-primitive log
+  unsigned int log_kept;            // records of the reduction under way
+  unsigned long long log_over;      // records that found the log full
 };
 
 // Tallies that every wave updates (global fields, counts) or that few keys
@@ -213,9 +216,9 @@ struct Tallies {
   uint32_t nrcv, nsamp, njobs;
   uint64_t nprim;
   // Log of finished paths' per-primitive entries (prim_add), reduced into
-  // `prim` by key after sorting (k_prim_reduce): record i is the key
-  // log_key[i] and the 10 fields' weights log_val[10 i ..]. log_n counts the
-  // records asked for, also past log_cap (those went to atomics).
+  // `prim` by key (k_prim_reduce): record i is the key log_key[i] and the 10
+  // fields' weights log_val[10 i ..]. log_n counts the records asked for, also
+  // past log_cap (those went to atomics).
   uint32_t* log_key;
   double* log_val;
   unsigned long long* log_n;
@@ -411,7 +414,7 @@ __device__ __forceinline__ unsigned long long wave_count_add(bool pred, unsigned
 // addresses, and the entries of a wave fall on as many primitives as it has
 // lanes, so the 20 atomics of an entry (x and x^2 per field) would cost far
 // more than the 84 bytes of a record in the log, which k_prim_reduce sums
-// by key after sorting. A full log takes the atomics. Must be called by the
+// by key. A full log takes the atomics. Must be called by the
 // whole wave.
 template <typename R>
 __device__ void prim_add(const Tallies& T, bool has, uint32_t key, const R* a, double factor) {
@@ -434,80 +437,7 @@ __device__ void prim_add(const Tallies& T, bool has, uint32_t key, const R* a, d
   }
 }
 
-// The sorted log (keys skey, record indices sidx, m records): each wave
-// takes PRIM_ROUNDS rounds of 64 consecutive records. While a round's
-// records all carry the key of the sums the wave holds, each lane adds its
-// record's x and x^2 of the 10 fields to its own sums; at a change of key
-// the sums are reduced across the wave and added with one set of 20
-// atomics, and a round of several keys reduces each of its runs of equal
-// keys so.
-constexpr uint32_t PRIM_ROUNDS = 8;
-
-__global__ void __launch_bounds__(256) k_prim_reduce(const uint32_t* __restrict__ skey,
-                                                     const uint32_t* __restrict__ sidx,
-                                                     const double* __restrict__ val, uint32_t m,
-                                                     double* prim, uint32_t mask_p, uint64_t nprim) {
-  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / 64u;
-  const uint32_t base = wave * 64u * PRIM_ROUNDS;
-  double* pb = prim + (size_t)(blockIdx.x & mask_p) * nprim * 40u;
-  double acc[20];
-#pragma unroll
-  for (int f = 0; f < 20; ++f) acc[f] = 0.0;
-  uint32_t acc_key = NONE;  // uniform over the wave: the key of acc
-  for (uint32_t r = 0; r < PRIM_ROUNDS; ++r) {
-    const uint32_t i = base + r * 64u + lane_id();
-    const bool in = i < m;
-    const uint64_t inmask = __ballot(in);
-    if (!inmask) break;  // lane 0 holds the round's first record from here on
-    const uint32_t key = in ? skey[i] : 0u;
-    double x[10];
-    if (in) {
-      const double2* v = (const double2*)(val + (size_t)sidx[i] * 10u);
-#pragma unroll
-      for (int f = 0; f < 5; ++f) {
-        const double2 t = v[f];
-        x[2 * f] = t.x;
-        x[2 * f + 1] = t.y;
-      }
-    } else {
-#pragma unroll
-      for (int f = 0; f < 10; ++f) x[f] = 0.0;
-    }
-    const uint32_t k0 = __shfl(key, 0, 64);
-    const bool one_key = __ballot(in && key == k0) == inmask;
-    if (!(one_key && k0 == acc_key) && acc_key != NONE) {
-      add_totals<20>(acc, pb + (size_t)acc_key * 20u);
-#pragma unroll
-      for (int f = 0; f < 20; ++f) acc[f] = 0.0;
-      acc_key = NONE;
-    }
-    if (one_key) {
-      acc_key = k0;
-#pragma unroll
-      for (int f = 0; f < 10; ++f) {
-        acc[2 * f] += x[f];
-        acc[2 * f + 1] += x[f] * x[f];
-      }
-      continue;
-    }
-    // several keys in the round: each run of equal keys on its own
-    bool todo = in;
-    for (uint64_t mask = __ballot(todo); mask; mask = __ballot(todo)) {
-      const int leader = __ffsll((unsigned long long)mask) - 1;
-      const uint32_t lkey = __shfl(key, leader, 64);
-      const bool match = todo && key == lkey;
-      double run[20];
-#pragma unroll
-      for (int f = 0; f < 10; ++f) {
-        run[2 * f] = match ? x[f] : 0.0;
-        run[2 * f + 1] = match ? x[f] * x[f] : 0.0;
-      }
-      add_totals<20>(run, pb + (size_t)lkey * 20u);
-      todo = todo && !match;
-    }
-  }
-  if (acc_key != NONE) add_totals<20>(acc, pb + (size_t)acc_key * 20u);
-}
+#include "ssolh_group.hpp"
 
 __global__ void k_iota32(uint32_t* a, uint32_t n) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1484,14 +1414,27 @@ __device__ __forceinline__ uint32_t start_key(const DScene& S, const SolveParams
   return job_of(prm, path) * ninst + inst;
 }
 
-// The start key of each of the wavefront's realisations and its index
+// The start key of realisation first + i
+template <bool FP32>
+struct StartKeyOf {
+  DScene S;
+  SolveParams prm;
+  uint64_t first;
+  uint32_t ninst;
+  __device__ uint32_t operator()(uint32_t i) const {
+    return start_key<FP32>(S, prm, first + i, ninst);
+  }
+};
+
+// The start keys of the wavefront's realisations and their indices, for the
+// radix sort
 template <bool FP32>
 __global__ void __launch_bounds__(256)
-k_start_keys(DScene S, SolveParams prm, uint64_t first, uint32_t count, uint32_t ninst,
-             uint32_t* __restrict__ key, uint32_t* __restrict__ idx) {
+k_start_keys(StartKeyOf<FP32> key_of, uint32_t count, uint32_t* __restrict__ key,
+             uint32_t* __restrict__ idx) {
   const uint32_t q = blockIdx.x * 256 + threadIdx.x;
   if (q >= count) return;
-  key[q] = start_key<FP32>(S, prm, first + q, ninst);
+  key[q] = key_of(q);
   idx[q] = q;
 }
 
@@ -1742,7 +1685,8 @@ struct ssolh_context {
   DevBuf start_sort;         // work bytes of the start-key sort
   DevBuf queue[2], list;     // paths in flight, their list
   DevBuf pend;               // pending entries
-  DevBuf counters, tallies, jobs, trace_ovf;
+  DevBuf tallies;            // counters, group counts, striped tallies, group offsets
+  DevBuf jobs, trace_ovf;
   // per-primitive log: keys, sorted keys, indices, sorted indices, values,
   // count, sort work (Tallies::log_*); log_sort, log_sidx, log_skey and
   // log_idx within it, log_sort_bytes of sort work
@@ -2045,8 +1989,8 @@ SSOLH_API int ssolh_destroy(ssolh_context* c) {
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   free_scene(c);
-  for (DevBuf* b : {&c->start_sort, &c->queue[0], &c->queue[1], &c->list, &c->pend, &c->counters,
-                    &c->tallies, &c->folded, &c->jobs, &c->trace_ovf, &c->lbvh, &c->render, &c->plog,
+  for (DevBuf* b : {&c->start_sort, &c->queue[0], &c->queue[1], &c->list, &c->pend, &c->tallies,
+                    &c->folded, &c->jobs, &c->trace_ovf, &c->lbvh, &c->render, &c->plog,
                     &c->adj_state, &c->adj_in, &c->adj_grad, &c->trk_vtx, &c->trk_type,
                     &c->trk_seq, &c->trk_count, &c->trk_pos})
     if (b->p) (void)hipFree(b->p);
@@ -2475,14 +2419,15 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
   if (!trk) c->trk_paths = 0;  // the recorded paths belong to the last solve only
   if (npend > MAX_PEND) { set_err("ssolh_solve: at most %d pending entries", MAX_PEND); return SSOLH_ERR_LIMIT; }
   // Tally layout: each tally is striped over up to 256 copies while its
-  // stripes hold at most 2^21 doubles; from the scratch array every stripe
+  // stripes hold at most 2^18 doubles (2^21 take 20 us more to clear and fold,
+  // and no flush is faster for them); from the scratch array every stripe
   // count is halved until all tallies take at most half of it.
   uint32_t sg, sr, ss, sx, sp;
   size_t n_global, n_rcv, n_samp, n_sxr, n_prim, n_u64, tally_bytes;
   for (size_t cap = 256;; cap >>= 1) {
     auto pow2_stripes = [cap](size_t per_stripe_doubles) {
       size_t k = cap;
-      while (k > 1 && k * per_stripe_doubles > (size_t(1) << 21)) k >>= 1;
+      while (k > 1 && k * per_stripe_doubles > (size_t(1) << 18)) k >>= 1;
       return (uint32_t)k;
     };
     sg = pow2_stripes((size_t)njobs * 16);
@@ -2535,7 +2480,7 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
     const uint64_t most = std::min<uint64_t>(std::min<uint64_t>(N, arena->size / per_slot), 1u << 28);
     HIP_TRY(start_sort_bytes((uint32_t)most, start_key_bits((uint64_t)njobs * c->ninstances),
                              c->stream, sort_bytes));
-    const size_t fixed = tally_bytes + (sort_bytes + 255) / 256 * 256 + (64u << 10);
+    const size_t fixed = tally_bytes + (sort_bytes + 255) / 256 * 256 + GROUP_BYTES + (64u << 10);
     const size_t rest = arena->size > fixed ? arena->size - fixed : 0;
     slots64 = rest / per_slot / BLOCK * BLOCK;
     if (slots64 < BLOCK) {
@@ -2579,10 +2524,29 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
   const size_t part = (n + 63) / 64 * 64;  // 256-byte aligned parts
   size_t sort_bytes = 0;
   int r = 0;
-  if (orderable) {
+  const bool group_starts = group_pays(slots, nkeys);
+  if (orderable && !group_starts) {
     HIP_TRY(start_sort_bytes(slots, key_bits, c->stream, sort_bytes));
     if ((r = alloc(c->start_sort, sort_bytes))) return r;
   }
+  // what a solve starts from zero, cleared at once: the counters, the record
+  // count of the log, the counts of the groupings by start key and by
+  // primitive (which each grouping leaves clear), the tallies (striped where
+  // many waves meet, see Tallies); beside them the groupings' offsets
+  // (the log's count, which waves add to, on a cache line of its own)
+  constexpr size_t head_bytes = 512;
+  static_assert(sizeof(Counters) <= 256, "head of the cleared buffer");
+  const size_t clear_bytes =
+      head_bytes + 2 * GROUP_KEYS * sizeof(uint32_t) + (tally_bytes + 15) / 16 * 16;
+  if ((r = alloc(c->tallies, clear_bytes + 2 * (GROUP_KEYS + 4) * sizeof(uint32_t)))) return r;
+  HIP_TRY(hipMemsetAsync(c->tallies.p, 0, clear_bytes, c->stream));
+  Counters* const ctr = (Counters*)c->tallies.p;
+  unsigned long long* const log_n = (unsigned long long*)((char*)c->tallies.p + 256);
+  uint32_t* const group = (uint32_t*)((char*)c->tallies.p + head_bytes);
+  uint32_t* const offsets = (uint32_t*)((char*)c->tallies.p + clear_bytes);
+  const GroupKeys start_keys{group, offsets, (uint32_t)std::min<uint64_t>(nkeys, UINT32_MAX)};
+  const GroupKeys prim_keys{group + GROUP_KEYS, offsets + GROUP_KEYS + 4,
+                            (uint32_t)std::min<uint64_t>((uint64_t)c->nprim * 2, UINT32_MAX)};
   // path queues, the list of places in the one being read, the waves' counts
   // of paths written and their scan
   for (int i = 0; i < 2; ++i)
@@ -2603,7 +2567,6 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
     W.pval = p + 2 * keys;
     W.qval = p + 2 * keys + vals;
   }
-  if ((r = alloc(c->counters, sizeof(Counters)))) return r;
   // traversal stack entries past the LDS ones, per lane of a launch
   if (ovf.extra) {
     ovf.stride = slots;
@@ -2670,9 +2633,7 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
                            njobs * sizeof(ssolh_sun), hipMemcpyHostToDevice, c->stream));
   }
 
-  // tallies (striped where many waves meet, see Tallies)
-  if ((r = alloc(c->tallies, tally_bytes))) return r;
-  double* tb = (double*)c->tallies.p;
+  double* tb = (double*)(group + 2 * GROUP_KEYS);
   c->T.global = tb;
   c->T.rcv = c->T.global + n_global;
   c->T.samp = c->T.rcv + n_rcv;
@@ -2688,10 +2649,9 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
   c->T.nsamp = c->nsamp;
   c->T.njobs = njobs;
   c->njobs = njobs;
-  HIP_TRY(hipMemsetAsync(c->tallies.p, 0, tally_bytes, c->stream));
-  HIP_TRY(hipMemsetAsync(c->counters.p, 0, sizeof(Counters), c->stream));
   // per-primitive log: room for one record per realisation, at most
-  // LOG_MAX_RECORDS (12.9 GB); none from the scratch array
+  // LOG_MAX_RECORDS; none from the scratch array
+  bool group_log = false;
   c->T.log_key = nullptr;
   c->T.log_val = nullptr;
   c->T.log_n = nullptr;
@@ -2703,14 +2663,16 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
     if (c->log_cap_test) cap = std::min(cap, c->log_cap_test);
     uint32_t bits = 1;
     while (bits < 32 && (uint64_t(1) << bits) < (uint64_t)c->nprim * 2) ++bits;
+    group_log = group_pays(cap, (uint64_t)c->nprim * 2);
     size_t sort_bytes = 0;
-    HIP_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, sort_bytes, (const uint32_t*)nullptr,
-                                               (uint32_t*)nullptr, (const uint32_t*)nullptr,
-                                               (uint32_t*)nullptr, (int)cap, 0, (int)bits,
-                                               c->stream));
+    if (!group_log)
+      HIP_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, sort_bytes, (const uint32_t*)nullptr,
+                                                 (uint32_t*)nullptr, (const uint32_t*)nullptr,
+                                                 (uint32_t*)nullptr, (int)cap, 0, (int)bits,
+                                                 c->stream));
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
     const size_t k4 = up((size_t)cap * 4);
-    const size_t bytes = 4 * k4 + up((size_t)cap * 80) + 256 + up(sort_bytes);
+    const size_t bytes = 4 * k4 + up((size_t)cap * 80) + up(sort_bytes);
     if (alloc(c->plog, bytes)) {
       // no room left beside the path state: every entry takes the atomics
       (void)hipGetLastError();
@@ -2724,22 +2686,46 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
       c->log_idx = (uint32_t*)(q + 2 * k4);
       c->log_sidx = (uint32_t*)(q + 3 * k4);
       c->T.log_val = (double*)(q + 4 * k4);
-      c->T.log_n = (unsigned long long*)(q + 4 * k4 + up((size_t)cap * 80));
-      c->log_sort = q + 4 * k4 + up((size_t)cap * 80) + 256;
+      c->T.log_n = log_n;
+      c->log_sort = q + 4 * k4 + up((size_t)cap * 80);
       c->log_sort_bytes = sort_bytes;
       c->log_key_bits = bits;
       c->T.log_cap = cap;
-      HIP_TRY(hipMemsetAsync(c->T.log_n, 0, sizeof(unsigned long long), c->stream));
     }
   }
   // Sums the logged records into the per-primitive tally and empties the
   // log
   auto log_flush = [&]() -> int {
     if (!c->T.log_cap) return 0;
+    const uint32_t cap = (uint32_t)c->T.log_cap;
+    // `shares` waves per key: one round of 64 records each for an even spread
+    // of m records, 131,072 waves at most for that. A flux map's peak holds
+    // several times the mean: with four rounds its waves run on alone (4e6
+    // records of 4,096 keys: 253 us, with one 200).
+    auto reduce = [&](uint32_t m, const uint32_t* skey) -> int {
+      const uint32_t shares = (uint32_t)std::max<uint64_t>(
+          1, std::min<uint64_t>(m / (64ull * prim_keys.keys), 131072u / prim_keys.keys));
+      const uint32_t blocks = (uint32_t)(((uint64_t)prim_keys.keys * shares + 3) / 4);
+      k_prim_reduce<<<blocks, 256, 0, c->stream>>>(prim_keys, skey, c->log_sidx, m, c->T.log_val,
+                                                   shares, c->T.prim);
+      HIP_TRY(hipGetLastError());
+      return 0;
+    };
+    if (group_log) {
+      k_group_rank<<<(cap + GROUP_BLOCK - 1) / GROUP_BLOCK, GROUP_THREADS, 0, c->stream>>>(
+          LogKeyOf{c->T.log_key}, c->T.log_n, cap, prim_keys, nullptr, c->log_skey);
+      HIP_TRY(hipGetLastError());
+      k_group_scan<<<1, GROUP_THREADS, 0, c->stream>>>(prim_keys, c->T.log_n, cap, &ctr->log_kept, ctr);
+      HIP_TRY(hipGetLastError());
+      k_group_place<<<(cap + 255) / 256, 256, 0, c->stream>>>(
+          c->T.log_key, c->log_skey, &ctr->log_kept, 0, prim_keys, c->log_sidx);
+      HIP_TRY(hipGetLastError());
+      return reduce(cap, nullptr);
+    }
     unsigned long long n = 0;
     HIP_TRY(hipMemcpyAsync(&n, c->T.log_n, sizeof(n), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    const uint32_t m = (uint32_t)std::min<unsigned long long>(n, c->T.log_cap);
+    const uint32_t m = (uint32_t)std::min<unsigned long long>(n, cap);
     c->log_overflowed += n - m;
     if (m) {
       ++c->log_flushes;
@@ -2749,10 +2735,7 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
       HIP_TRY(hipcub::DeviceRadixSort::SortPairs(c->log_sort, sb, c->T.log_key, c->log_skey,
                                                  c->log_idx, c->log_sidx, (int)m, 0,
                                                  (int)c->log_key_bits, c->stream));
-      const uint32_t per_block = 256 * PRIM_ROUNDS;
-      k_prim_reduce<<<(m + per_block - 1) / per_block, 256, 0, c->stream>>>(
-          c->log_skey, c->log_sidx, c->T.log_val, m, c->T.prim, c->T.mask_p, c->T.nprim);
-      HIP_TRY(hipGetLastError());
+      if (int e = reduce(m, c->log_skey)) return e;
     }
     if (n) HIP_TRY(hipMemsetAsync(c->T.log_n, 0, sizeof(unsigned long long), c->stream));
     return 0;
@@ -2770,7 +2753,6 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
   prm.job_suns = job_suns_h ? (const ssolh_sun*)((char*)c->jobs.p + (njobs + 1) * sizeof(uint64_t))
                             : nullptr;
 
-  Counters* ctr = (Counters*)c->counters.p;
   PathArgs args{};
   args.S = c->scn;
   args.SQ = c->shapeq;
@@ -2817,12 +2799,26 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
     uint32_t* key = (uint32_t*)c->queue[1].p;
     uint32_t *skey = key + part, *idx = skey + part, *order = idx + part;
     const uint32_t gg = (count + 255) / 256;
+    const StartKeyOf<false> k64{c->scn, prm, first, c->ninstances};
+    const StartKeyOf<true> k32{c->scn, prm, first, c->ninstances};
+    if (group_starts) {
+      const uint32_t gb = (count + GROUP_BLOCK - 1) / GROUP_BLOCK;
+      if (fp32)
+        k_group_rank<<<gb, GROUP_THREADS, 0, c->stream>>>(k32, nullptr, count, start_keys, key, skey);
+      else
+        k_group_rank<<<gb, GROUP_THREADS, 0, c->stream>>>(k64, nullptr, count, start_keys, key, skey);
+      HIP_TRY(hipGetLastError());
+      k_group_scan<<<1, GROUP_THREADS, 0, c->stream>>>(start_keys, nullptr, 0, nullptr, nullptr);
+      HIP_TRY(hipGetLastError());
+      k_group_place<<<gg, 256, 0, c->stream>>>(key, skey, nullptr, count, start_keys, order);
+      HIP_TRY(hipGetLastError());
+      args.order = order;
+      return 0;
+    }
     if (fp32)
-      k_start_keys<true><<<gg, 256, 0, c->stream>>>(c->scn, prm, first, count, c->ninstances, key,
-                                                     idx);
+      k_start_keys<<<gg, 256, 0, c->stream>>>(k32, count, key, idx);
     else
-      k_start_keys<false><<<gg, 256, 0, c->stream>>>(c->scn, prm, first, count, c->ninstances,
-                                                      key, idx);
+      k_start_keys<<<gg, 256, 0, c->stream>>>(k64, count, key, idx);
     HIP_TRY(hipGetLastError());
     size_t sb = sort_bytes;
     HIP_TRY(hipcub::DeviceRadixSort::SortPairs(c->start_sort.p, sb, key, skey, idx, order,
@@ -2882,14 +2878,13 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
       if ((r = resume(going))) return r;
     } while (!run_through(going));
     HIP_TRY(hipEventRecord(c->ev[2], c->stream));
-    if (c->T.log_cap) {
-      if ((r = log_flush())) return r;
-    } else {
-      HIP_TRY(hipStreamSynchronize(c->stream));
+    if ((r = log_flush())) return r;
+    if (first + slots < N) {  // the last chunk's events are read when the solve ends
+      HIP_TRY(hipEventSynchronize(c->ev[2]));
+      float t = 0;
+      (void)hipEventElapsedTime(&t, c->ev[1], c->ev[2]);
+      ms_path += t;
     }
-    float t = 0;
-    (void)hipEventElapsedTime(&t, c->ev[1], c->ev[2]);
-    ms_path += t;
   }
   // fold the stripes: into one buffer, copied whole to pinned host memory;
   // from the scratch array, in place
@@ -2951,6 +2946,9 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
   HIP_TRY(hipEventRecord(c->ev[3], c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
   (void)hipEventElapsedTime(&total_ms, c->ev[0], c->ev[3]);
+  float last_ms = 0;
+  (void)hipEventElapsedTime(&last_ms, c->ev[1], c->ev[2]);
+  ms_path += last_ms;
   double rays = 0;  // counted beside job 0's global fields
   if (c->staged) {
     memcpy(&c->last, c->stage, sizeof(Counters));
@@ -2960,6 +2958,8 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
     HIP_TRY(hipMemcpy(&rays, c->F.global + 13, sizeof(rays), hipMemcpyDeviceToHost));
   }
   c->segments = (uint64_t)rays;
+  c->log_flushes += c->last.log_flushes;
+  c->log_overflowed += c->last.log_over;
   if (trk) HIP_TRY(hipMemcpy(&c->trk_nvtx, c->trk_count.p, sizeof(c->trk_nvtx), hipMemcpyDeviceToHost));
   c->kernel_ms = total_ms;
   c->trace_ms = ms_path;  // tracing and shading are one kernel
@@ -3018,8 +3018,8 @@ SSOLH_API int ssolh_solve_noalloc(ssolh_context* c, const struct ssolh_solve_arg
   // The solve's buffers come from the scratch array: the context's own
   // buffers are set aside for the call (nothing is freed or allocated) and
   // put back after it.
-  DevBuf* bufs[] = {&c->start_sort, &c->queue[0], &c->queue[1], &c->list,
-                    &c->pend,       &c->counters, &c->tallies,  &c->trace_ovf};
+  DevBuf* bufs[] = {&c->start_sort, &c->queue[0], &c->queue[1], &c->list, &c->pend,
+                    &c->tallies,    &c->trace_ovf};
   constexpr size_t NB = sizeof(bufs) / sizeof(bufs[0]);
   DevBuf saved[NB];
   for (size_t i = 0; i < NB; ++i) {
@@ -3254,6 +3254,38 @@ SSOLH_API int ssolh_test_threefry(ssolh_context* c, uint32_t n, const uint64_t* 
   HIP_TRY(hipMemcpy(out, d_o, n * 32, hipMemcpyDeviceToHost));
   (void)hipFree(d_c); (void)hipFree(d_k); (void)hipFree(d_o);
   return 0;
+}
+
+SSOLH_API int ssolh_test_group(ssolh_context* c, uint32_t n, uint32_t nkeys, const uint32_t* key,
+                               uint32_t* order, uint32_t* offsets) {
+  if (!c || !n || !nkeys || nkeys > GROUP_KEYS || !key || !order || !offsets) return SSOLH_ERR_ARG;
+  for (uint32_t i = 0; i < n; ++i)
+    if (key[i] >= nkeys) return SSOLH_ERR_ARG;
+  HIP_TRY(hipSetDevice(c->device));
+  DevBuf keys, work;
+  int r = dev_alloc(keys, 3 * (size_t)n * 4);
+  if (!r) r = dev_alloc(work, GROUP_BYTES / 2);
+  const auto run = [&]() -> int {
+    uint32_t *d_key = (uint32_t*)keys.p, *d_rank = d_key + n, *d_order = d_rank + n;
+    const GroupKeys g{(uint32_t*)work.p, (uint32_t*)work.p + GROUP_KEYS, nkeys};
+    HIP_TRY(hipMemsetAsync(work.p, 0, GROUP_KEYS * 4, c->stream));
+    HIP_TRY(hipMemcpyAsync(d_key, key, (size_t)n * 4, hipMemcpyHostToDevice, c->stream));
+    k_group_rank<<<(n + GROUP_BLOCK - 1) / GROUP_BLOCK, GROUP_THREADS, 0, c->stream>>>(
+        LogKeyOf{d_key}, nullptr, n, g, nullptr, d_rank);
+    HIP_TRY(hipGetLastError());
+    k_group_scan<<<1, GROUP_THREADS, 0, c->stream>>>(g, nullptr, 0, nullptr, nullptr);
+    HIP_TRY(hipGetLastError());
+    k_group_place<<<(n + 255) / 256, 256, 0, c->stream>>>(d_key, d_rank, nullptr, n, g, d_order);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    HIP_TRY(hipMemcpy(order, d_order, (size_t)n * 4, hipMemcpyDeviceToHost));
+    HIP_TRY(hipMemcpy(offsets, g.offsets, ((size_t)nkeys + 1) * 4, hipMemcpyDeviceToHost));
+    return 0;
+  };
+  if (!r) r = run();
+  (void)hipFree(keys.p);
+  (void)hipFree(work.p);
+  return r;
 }
 
 SSOLH_API int ssolh_test_wave_sum(ssolh_context* c, uint32_t nwaves, const double* in,
