@@ -8,6 +8,7 @@
 #include <map>
 #include <memory>
 #include <string>
+#include <mutex>
 #include <vector>
 
 #include "ssol.h"
@@ -29,6 +30,24 @@ struct ssol_refcounted {
 
 struct solve_cache;  // flattened scene of the last solve (ssol_solve.cpp)
 
+// Memory of an estimator's tallies, not cleared
+struct tally_block {
+  std::unique_ptr<uint64_t[]> mem;
+  size_t words = 0;
+};
+
+// Blocks of released estimators for the device's next solves: the tallies of
+// 10,000 heliostats are 3.6 MB, whose fresh pages cost more than the copy into
+// them. At most SPARE_BLOCKS blocks of SPARE_WORDS words in all, freed with
+// the device.
+struct tally_spares {
+  static constexpr size_t SPARE_BLOCKS = 2, SPARE_WORDS = size_t(4) << 20;
+  std::mutex mutex;
+  std::vector<tally_block> blocks;
+  tally_block take(size_t words);
+  void give(tally_block&& b);
+};
+
 struct ssol_device : ssol_refcounted {
   int verbose = 0;
   unsigned nthreads = 1;
@@ -37,6 +56,7 @@ struct ssol_device : ssol_refcounted {
   unsigned graph_iterations = 0;  // 0: host-driven wavefront iterations
   ssolh_context* gpu = nullptr;  // created at the first solve
   solve_cache* cache = nullptr;
+  tally_spares spares;
 };
 
 struct ssol_spectrum : ssol_refcounted {
@@ -150,18 +170,23 @@ struct estimator_shape_block {
   size_t first;  // per-primitive slot of triangle 0
 };
 
+// Where a scene's tallies lie; shared by the estimators of its solves
+struct tally_slots {
+  std::map<uint32_t, int> rcv;   // instance id -> receiver slot
+  std::map<uint32_t, int> samp;  // instance id -> sampled slot
+  std::map<std::pair<uint32_t, uint32_t>, size_t> prim_first;  // (inst id, shape uid)
+};
+
 struct ssol_estimator : ssol_refcounted {
   ssol_device* dev = nullptr;
   size_t realisation_count = 0;
   size_t failed_count = 0;
   double sampled_area = 0;
   double global[6][2] = {};
-  std::vector<double> rcv, samp, sxr, prim;
-  std::vector<uint64_t> samp_count;
-  std::map<uint32_t, int> rcv_slot;   // instance id -> receiver slot
-  std::map<uint32_t, int> samp_slot;  // instance id -> sampled slot
-  std::map<uint32_t, int> rcv_mask;   // instance id -> receiver mask
-  std::map<std::pair<uint32_t, uint32_t>, size_t> prim_first;  // (inst id, shape uid)
+  tally_block block;  // holds the five arrays
+  double *rcv = nullptr, *samp = nullptr, *sxr = nullptr, *prim = nullptr;
+  uint64_t* samp_count = nullptr;
+  std::shared_ptr<const tally_slots> slots;
   size_t nrcv = 0, nsamp = 0;
   ssp_rng* rng = nullptr;
   ssol_solve_stats stats = {};

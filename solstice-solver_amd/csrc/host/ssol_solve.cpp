@@ -432,12 +432,41 @@ void frame(const double* d, double* m) {
 }
 
 struct Layout {
-  std::vector<int> rcv_slot, samp_slot;
-  std::map<std::pair<uint32_t, uint32_t>, size_t> prim_first;
+  std::shared_ptr<tally_slots> slots = std::make_shared<tally_slots>();
   size_t nrcv = 0, nsamp = 0, nprim = 0;
 };
 
-void push_data_sig(std::vector<uint64_t>& sig, const ssol_data& d) {
+// A signature taken word by word against the one of the last solve, which it
+// copies only from the first word that differs
+class Signature {
+ public:
+  explicit Signature(const std::vector<uint64_t>* last) : last_(last) {}
+  void push_back(uint64_t x) {
+    if (same_) {
+      if (last_ && at_ < last_->size() && (*last_)[at_] == x) { ++at_; return; }
+      differ();
+    }
+    words_.push_back(x);
+  }
+  bool unchanged() const { return same_ && last_ && at_ == last_->size(); }
+  // the words of a changed signature
+  std::vector<uint64_t>& words() {
+    if (same_) differ();
+    return words_;
+  }
+
+ private:
+  void differ() {
+    same_ = false;
+    if (last_) words_.assign(last_->begin(), last_->begin() + at_);
+  }
+  const std::vector<uint64_t>* last_;
+  std::vector<uint64_t> words_;
+  size_t at_ = 0;
+  bool same_ = true;
+};
+
+void push_data_sig(Signature& sig, const ssol_data& d) {
   sig.push_back((uint64_t)d.type);
   if (d.type == SSOL_DATA_REAL) {
     uint64_t b;
@@ -449,7 +478,7 @@ void push_data_sig(std::vector<uint64_t>& sig, const ssol_data& d) {
   }
 }
 
-void push_medium_sig(std::vector<uint64_t>& sig, const ssol_medium& m) {
+void push_medium_sig(Signature& sig, const ssol_medium& m) {
   push_data_sig(sig, m.extinction);
   push_data_sig(sig, m.refractive_index);
 }
@@ -459,7 +488,7 @@ void push_medium_sig(std::vector<uint64_t>& sig, const ssol_medium& m) {
 // anywhere else), which a client may rewrite between solves without any
 // setter call, so the baked constants are checked against a fresh
 // evaluation on every solve
-void push_shader_sig(std::vector<uint64_t>& sig, const ssol_material* m,
+void push_shader_sig(Signature& sig, const ssol_material* m,
                      const std::vector<double>& wls) {
   auto push = [&](double v) {
     uint64_t b;
@@ -486,11 +515,10 @@ void push_shader_sig(std::vector<uint64_t>& sig, const ssol_material* m,
 
 // Everything flatten() reads, so that an unchanged scene is not flattened
 // and uploaded again
-// Instance transforms go to *xf, the rest to the returned signature: scenes
-// that differ only in *xf share their objects, sampling and tally layout.
-std::vector<uint64_t> scene_signature(const ssol_scene* scn, std::vector<uint64_t>* xf) {
-  std::vector<uint64_t> sig;
-  xf->clear();
+// Instance transforms go to xf, the rest to sig: scenes that differ only in
+// xf share their objects, sampling and tally layout. An object is walked once,
+// however many instances share it.
+void scene_signature(const ssol_scene* scn, Signature& sig, Signature& xf) {
   auto P = [&](const void* p) { sig.push_back((uint64_t)(uintptr_t)p); };
   P(scn);
   P(scn->sun);
@@ -502,21 +530,27 @@ std::vector<uint64_t> scene_signature(const ssol_scene* scn, std::vector<uint64_
     sig.push_back(scn->atmosphere->gen);
     push_data_sig(sig, scn->atmosphere->extinction);
   }
-  std::vector<const ssol_material*> mats;
+  std::vector<const ssol_object*> objects;
   for (const ssol_instance* in : scn->instances) {
     P(in);
     sig.push_back(in->id);
     for (int k = 0; k < 12; ++k) {
       uint64_t b;
       memcpy(&b, &in->transform[k], 8);
-      xf->push_back(b);
+      xf.push_back(b);
     }
     sig.push_back((uint64_t)in->receiver_mask);
     sig.push_back((uint64_t)in->per_primitive);
     sig.push_back((uint64_t)in->sample);
     P(in->object);
-    sig.push_back(in->object->sshapes.size());
-    for (const shaded_shape& ss : in->object->sshapes) {
+    if (objects.empty() || objects.back() != in->object) objects.push_back(in->object);
+  }
+  std::sort(objects.begin(), objects.end());
+  objects.erase(std::unique(objects.begin(), objects.end()), objects.end());
+  std::vector<const ssol_material*> mats;
+  for (const ssol_object* o : objects) {
+    sig.push_back(o->sshapes.size());
+    for (const shaded_shape& ss : o->sshapes) {
       P(ss.shape);
       sig.push_back(ss.shape->gen);
       for (const ssol_material* m : {ss.front, ss.back}) {
@@ -536,7 +570,6 @@ std::vector<uint64_t> scene_signature(const ssol_scene* scn, std::vector<uint64_
     for (const ssol_material* m : mats)
       if (m->type != SSOL_MATERIAL_VIRTUAL) push_shader_sig(sig, m, wls);
   }
-  return sig;
 }
 
 // Device form of a sun (src/ssol_sun.c:214-279). With add_spectrum false
@@ -696,8 +729,8 @@ res_T flatten(ssol_scene* scn, Flat& f, Layout& L) {
     d.sampled = in->sample ? (int32_t)L.nsamp++ : -1;
     d.isshape_first = (uint32_t)f.isshapes.size();
     d.user_id = in->id;
-    L.rcv_slot.push_back(d.receiver);
-    L.samp_slot.push_back(d.sampled);
+    if (d.receiver >= 0) L.slots->rcv[in->id] = d.receiver;
+    if (d.sampled >= 0) L.slots->samp[in->id] = d.sampled;
     if (in->receiver_mask) has_receiver = true;
     std::vector<ssolh_inst_sshape> frames(in->object->sshapes.size());
     instance_frames(in, d, frames.data());
@@ -707,7 +740,7 @@ res_T flatten(ssol_scene* scn, Flat& f, Layout& L) {
       is.prim_tally = -1;
       if (in->receiver_mask && in->per_primitive) {
         is.prim_tally = (int64_t)L.nprim;
-        L.prim_first[{in->id, sh->uid}] = L.nprim;
+        L.slots->prim_first[{in->id, sh->uid}] = L.nprim;
         L.nprim += sh->ids.size() / 3;
       }
       f.isshapes.push_back(is);
@@ -802,6 +835,7 @@ void mc_result(double w, double w2, double N, ssol_mc_result* r) {
 void estimator_release(ssol_estimator* e) {
   if (e->rng) ssp_rng_ref_put(e->rng);
   ssol_device* d = e->dev;
+  d->spares.give(std::move(e->block));
   delete e;
   device_ref_put_(d);
 }
@@ -823,6 +857,33 @@ struct solve_cache {
   Layout layout;
 };
 
+tally_block tally_spares::take(size_t words) {
+  {
+    const std::lock_guard<std::mutex> lock(mutex);
+    for (size_t i = 0; i < blocks.size(); ++i) {
+      if (blocks[i].words < words) continue;
+      tally_block b = std::move(blocks[i]);
+      blocks.erase(blocks.begin() + i);
+      return b;
+    }
+  }
+  tally_block b;
+  b.mem.reset(new uint64_t[words]);
+  b.words = words;
+  return b;
+}
+
+void tally_spares::give(tally_block&& b) {
+  if (!b.words || b.words > SPARE_WORDS) return;
+  const std::lock_guard<std::mutex> lock(mutex);
+  blocks.push_back(std::move(b));
+  // the oldest leave
+  size_t words = 0, n = blocks.size();
+  while (n && blocks.size() - n < SPARE_BLOCKS && words + blocks[n - 1].words <= SPARE_WORDS)
+    words += blocks[--n].words;
+  blocks.erase(blocks.begin(), blocks.begin() + n);
+}
+
 namespace ssol {
 void solve_cache_free(ssol_device* d) {
   delete d->cache;
@@ -837,10 +898,18 @@ namespace {
 // generation stamp), creates the GPU context at the first solve.
 res_T prepare_scene(ssol_scene* scn) {
   ssol_device* dev = scn->dev;
-  std::vector<uint64_t> xf;
-  std::vector<uint64_t> sig = scene_signature(scn, &xf);
-  const bool same = dev->cache && dev->cache->sig == sig;
-  const bool cached = same && dev->cache->xf == xf;
+  bool same, cached;
+  std::vector<uint64_t> sig, xf;  // of a changed scene
+  {
+    Signature s(dev->cache ? &dev->cache->sig : nullptr), x(dev->cache ? &dev->cache->xf : nullptr);
+    scene_signature(scn, s, x);
+    same = s.unchanged();
+    cached = same && x.unchanged();
+    if (!cached) {
+      sig = same ? dev->cache->sig : std::move(s.words());
+      xf = x.unchanged() ? dev->cache->xf : std::move(x.words());
+    }
+  }
   if (!same) {
     solve_cache_free(dev);
     dev->cache = new solve_cache();
@@ -1039,17 +1108,20 @@ res_T ssol_solve(struct ssol_scene* scn, const struct ssp_rng* rng, const size_t
   }
   est->nrcv = L.nrcv;
   est->nsamp = L.nsamp;
-  est->rcv.assign(L.nrcv * 40, 0);
-  est->samp.assign(L.nsamp * 4, 0);
-  est->samp_count.assign(L.nsamp, 0);
-  est->sxr.assign(L.nsamp * L.nrcv * 40, 0);
-  est->prim.assign(L.nprim * 40, 0);
+  est->slots = L.slots;
+  const size_t nsxr = L.nsamp * L.nrcv * 40;
+  est->block = dev->spares.take(L.nrcv * 40 + L.nsamp * 5 + nsxr + L.nprim * 40);
+  est->rcv = (double*)est->block.mem.get();
+  est->samp = est->rcv + L.nrcv * 40;
+  est->sxr = est->samp + L.nsamp * 4;
+  est->prim = est->sxr + nsxr;
+  est->samp_count = (uint64_t*)(est->prim + L.nprim * 40);
   ssolh_tallies t{};
-  t.receivers = est->rcv.data();
-  t.sampled = est->samp.data();
-  t.sampled_count = (uint64_t*)est->samp_count.data();
-  t.sampled_x_receivers = est->sxr.data();
-  t.primitives = est->prim.data();
+  t.receivers = est->rcv;
+  t.sampled = est->samp;
+  t.sampled_count = est->samp_count;
+  t.sampled_x_receivers = est->sxr;
+  t.primitives = est->prim;
   e = ssolh_tallies_download(dev->gpu, &t);
   if (e) {
     fprintf(stderr, "ssol_solve: tally download failed: %s\n", ssolh_last_error());
@@ -1060,12 +1132,6 @@ res_T ssol_solve(struct ssol_scene* scn, const struct ssp_rng* rng, const size_t
   est->realisation_count = t.realisation_count;
   est->failed_count = t.failed_count;
   est->sampled_area = f.scn.sampled_area;
-  for (size_t i = 0; i < scn->instances.size(); ++i) {
-    const ssol_instance* in = scn->instances[i];
-    if (L.rcv_slot[i] >= 0) est->rcv_slot[in->id] = L.rcv_slot[i];
-    if (L.samp_slot[i] >= 0) est->samp_slot[in->id] = L.samp_slot[i];
-  }
-  est->prim_first = L.prim_first;
   est->stats.segments = t.segments;
   est->stats.paths = N;
   est->stats.pending_spills = t.pending_spills;
@@ -1114,8 +1180,8 @@ res_T ssol_estimator_get_mc_receiver(struct ssol_estimator* e, const struct ssol
                                      const enum ssol_side_flag side, struct ssol_mc_receiver* rcv) {
   if (!e || !inst || !rcv || !(inst->receiver_mask & (int)side)) return RES_BAD_ARG;
   memset(rcv, 0, sizeof(*rcv));
-  auto it = e->rcv_slot.find(inst->id);
-  if (it == e->rcv_slot.end()) return RES_OK;
+  auto it = e->slots->rcv.find(inst->id);
+  if (it == e->slots->rcv.end()) return RES_OK;
   const int s = side == SSOL_FRONT ? 0 : 1;
   fill_receiver(&e->rcv[((size_t)it->second * 2 + s) * 20], (double)e->realisation_count, rcv);
   e->refs.push_back(std::unique_ptr<ssol_estimator::rcv_ref>(
@@ -1135,10 +1201,10 @@ res_T ssol_estimator_get_mc_sampled_x_receiver(struct ssol_estimator* e,
       !(ri->receiver_mask & (int)side))
     return RES_BAD_ARG;
   memset(rcv, 0, sizeof(*rcv));
-  auto si = e->samp_slot.find(samp->id);
-  if (si == e->samp_slot.end()) return RES_BAD_ARG;
-  auto it = e->rcv_slot.find(ri->id);
-  if (it == e->rcv_slot.end()) return RES_OK;
+  auto si = e->slots->samp.find(samp->id);
+  if (si == e->slots->samp.end()) return RES_BAD_ARG;
+  auto it = e->slots->rcv.find(ri->id);
+  if (it == e->slots->rcv.end()) return RES_OK;
   const int s = side == SSOL_FRONT ? 0 : 1;
   const size_t key = ((size_t)si->second * e->nrcv + (size_t)it->second) * 2 + (size_t)s;
   fill_receiver(&e->sxr[key * 20], (double)e->realisation_count, rcv);
@@ -1176,8 +1242,8 @@ res_T ssol_estimator_get_sampled_count(const struct ssol_estimator* e, size_t* n
 res_T ssol_estimator_get_mc_sampled(struct ssol_estimator* e, const struct ssol_instance* inst,
                                     struct ssol_mc_sampled* s) {
   if (!e || !inst || !s) return RES_BAD_ARG;
-  auto it = e->samp_slot.find(inst->id);
-  if (it == e->samp_slot.end()) return RES_BAD_ARG;
+  auto it = e->slots->samp.find(inst->id);
+  if (it == e->slots->samp.end()) return RES_BAD_ARG;
   const double* b = &e->samp[(size_t)it->second * 4];
   s->nb_samples = e->samp_count[it->second];
   mc_result(b[0], b[1], (double)s->nb_samples, &s->cos_factor);
@@ -1237,8 +1303,8 @@ res_T ssol_mc_receiver_get_mc_shape(struct ssol_mc_receiver* rcv, const struct s
   mc->N__ = rcv->N__;
   mc->shape__ = shape;
   mc->mc__ = nullptr;
-  auto it = e->prim_first.find({inst->id, shape->uid});
-  if (it != e->prim_first.end() && ref->slot >= 0) {
+  auto it = e->slots->prim_first.find({inst->id, shape->uid});
+  if (it != e->slots->prim_first.end() && ref->slot >= 0) {
     e->shape_refs.push_back(std::unique_ptr<ssol_estimator::shape_ref>(
         new ssol_estimator::shape_ref{e, it->second * 2 + (size_t)ref->side, shape}));
     mc->mc__ = e->shape_refs.back().get();
@@ -1382,17 +1448,17 @@ res_T ssol_solve_adjoint(struct ssol_scene* scn, const struct ssp_rng* rng, cons
   // parameter slot of every scene instance (flat instances follow the
   // scene's instance order)
   std::vector<int32_t> inst_param(scn->instances.size(), -1);
+  std::unordered_map<const ssol_instance*, size_t> index;
+  for (size_t i = 0; i < scn->instances.size(); ++i) index.emplace(scn->instances[i], i);
   for (size_t p = 0; p < nparams; ++p) {
-    const ssol_instance* h = heliostats[p];
-    size_t i = 0;
-    while (i < scn->instances.size() && scn->instances[i] != h) ++i;
-    if (i == scn->instances.size() || inst_param[i] >= 0) return RES_BAD_ARG;
-    inst_param[i] = (int32_t)p;
+    const auto it = index.find(heliostats[p]);
+    if (it == index.end() || inst_param[it->second] >= 0) return RES_BAD_ARG;
+    inst_param[it->second] = (int32_t)p;
   }
   std::vector<double> gmap;
   if (d_map) {
-    auto it = L.prim_first.find({map_receiver->id, map_shape->uid});
-    if (it == L.prim_first.end()) {
+    auto it = L.slots->prim_first.find({map_receiver->id, map_shape->uid});
+    if (it == L.slots->prim_first.end()) {
       log_error(dev, "ssol_solve_adjoint: the map shape has no per-primitive tallies.\n");
       return RES_BAD_ARG;
     }
