@@ -409,6 +409,17 @@ __device__ __forceinline__ unsigned long long wave_count_add(bool pred, unsigned
   return base + (unsigned long long)__popcll(below);
 }
 
+// Record `pos` of the per-primitive log: the weights a[f] * factor of a key
+template <typename R>
+__device__ __forceinline__ void log_record(const Tallies& T, uint64_t pos, uint32_t key, const R* a,
+                                           double factor) {
+  T.log_key[pos] = key;
+  double2* v = (double2*)(T.log_val + pos * 10u);
+#pragma unroll
+  for (int f = 0; f < 5; ++f)
+    v[f] = make_double2((double)a[2 * f] * factor, (double)a[2 * f + 1] * factor);
+}
+
 // A finished path's per-primitive entry: the key and the 10 fields' weights
 // a[f] * factor. FP64 atomics issue at one device-wide rate whatever their
 // addresses, and the entries of a wave fall on as many primitives as it has
@@ -421,11 +432,7 @@ __device__ void prim_add(const Tallies& T, bool has, uint32_t key, const R* a, d
   const unsigned long long pos = T.log_cap ? wave_count_add(has, T.log_n) : ~0ull;
   if (!has) return;
   if (pos < T.log_cap) {
-    T.log_key[pos] = key;
-    double2* v = (double2*)(T.log_val + pos * 10u);
-#pragma unroll
-    for (int f = 0; f < 5; ++f)
-      v[f] = make_double2((double)a[2 * f] * factor, (double)a[2 * f + 1] * factor);
+    log_record(T, pos, key, a, factor);
     return;
   }
   double* pb = T.prim + (size_t)(blockIdx.x & T.mask_p) * T.nprim * 40u + (size_t)key * 20u;
@@ -2649,8 +2656,9 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
   c->T.nsamp = c->nsamp;
   c->T.njobs = njobs;
   c->njobs = njobs;
-  // per-primitive log: room for one record per realisation, at most
-  // LOG_MAX_RECORDS; none from the scratch array
+  // per-primitive log: room for one record per realisation, or four where
+  // receivers pass light on and a path logs each primitive it met (a cavity
+  // of ten bounces: 3.2), at most LOG_MAX_RECORDS; none from the scratch array
   bool group_log = false;
   c->T.log_key = nullptr;
   c->T.log_val = nullptr;
@@ -2659,7 +2667,8 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
   c->log_flushes = 0;
   c->log_overflowed = 0;
   if (!arena && c->nprim) {
-    uint32_t cap = (uint32_t)std::min<uint64_t>(N, LOG_MAX_RECORDS);
+    uint32_t cap = (uint32_t)std::min<uint64_t>(
+        std::min<uint64_t>(N, LOG_MAX_RECORDS) * (c->may_pend ? 4 : 1), LOG_MAX_RECORDS);
     if (c->log_cap_test) cap = std::min(cap, c->log_cap_test);
     uint32_t bits = 1;
     while (bits < 32 && (uint64_t(1) << bits) < (uint64_t)c->nprim * 2) ++bits;

@@ -75,13 +75,20 @@ struct PathQ {
 };
 
 // Pending entries of the wavefront's realisations (receivers hit in
-// passing), by slot: key and ten weights of entry k at k * slots + slot;
+// passing): key and ten weights of entry k of a slot at slot * npend + k;
 // Path::npk, nqk count the entries in use. The weights are of the form's
-// type.
+// type. Bound by the lines they touch: the paths of a wave hold ever sparser
+// slots, so an entry's weights lie side by side (80 or 40 bytes, one or two
+// lines) and not by weight, where each of the ten would be a line of its own.
 struct Pending {
-  uint32_t *pkey, *qkey;   // receiver, per-primitive keys
-  void *pval, *qval;       // [entry][10][slots]
+  uint32_t *pkey, *qkey;   // receiver, per-primitive keys: [slot][entry]
+  void *pval, *qval;       // [slot][entry][10]
   uint32_t npend;
+};
+// Two neighbouring weights of an entry
+template <typename R>
+struct alignas(2 * sizeof(R)) WeightPair {
+  R a, b;
 };
 
 struct PathArgs {
@@ -298,19 +305,26 @@ __device__ __forceinline__ void receiver_weights(R in0, R in1, R in2, R kabs, R 
   w[8] = (in2 - in0) * kabs; w[9] = (in1 - in0) * kabs;
 }
 
-// Add the weights of a hit to the path's pending entries (n of them in use);
-// false when npend entries hold other keys.
+// Add the weights of a hit to the path's pending entries (n of the npend at
+// keys, vals in use); false when npend entries hold other keys.
 template <typename R>
-__device__ bool pend_add(uint32_t* keys, R* vals, size_t stride, uint32_t npend, uint32_t& n,
-                         uint32_t key, const R* w) {
+__device__ bool pend_add(uint32_t* keys, R* vals, uint32_t npend, uint32_t& n, uint32_t key,
+                         const R* w) {
   for (uint32_t k = 0; k < n; ++k) {
-    if (keys[k * stride] != key) continue;
-    for (int f = 0; f < 10; ++f) vals[((size_t)k * 10 + f) * stride] += w[f];
+    if (keys[k] != key) continue;
+    auto* v = (WeightPair<R>*)(vals + k * 10);
+#pragma unroll
+    for (int f = 0; f < 5; ++f) {
+      const WeightPair<R> x = v[f];
+      v[f] = {x.a + w[2 * f], x.b + w[2 * f + 1]};
+    }
     return true;
   }
   if (n >= npend) return false;
-  keys[n * stride] = key;
-  for (int f = 0; f < 10; ++f) vals[((size_t)n * 10 + f) * stride] = w[f];
+  keys[n] = key;
+  auto* v = (WeightPair<R>*)(vals + n * 10);
+#pragma unroll
+  for (int f = 0; f < 5; ++f) v[f] = {w[2 * f], w[2 * f + 1]};
   ++n;
   return true;
 }
@@ -324,6 +338,20 @@ __device__ void spill(double* base, uint64_t key, const R* w, unsigned long long
     atomic_add(base + key * 20 + 2 * f, x);
     atomic_add(base + key * 20 + 2 * f + 1, x * x);
   }
+}
+
+// The same of a primitive, through the log (see prim_add; any lanes may call)
+template <typename R>
+__device__ void spill_prim(const Tallies& T, uint32_t key, const R* w, unsigned long long* spills) {
+  if (T.log_cap) {
+    const unsigned long long pos = atomicAdd(T.log_n, 1ull);
+    if (pos < T.log_cap) {
+      atomicAdd(spills, 1ull);
+      log_record(T, pos, key, w, 1.0);
+      return;
+    }
+  }
+  spill(T.prim + (size_t)(blockIdx.x & T.mask_p) * T.nprim * 40u, key, w, spills);
 }
 
 // The point a ray hit, relative to its origin's frame, and the unit normal
@@ -373,7 +401,6 @@ __device__ __forceinline__ bool shade_path(const PathArgs& a, Path<F>& p,
   using vec = typename F::vec;
   const DScene& S = a.S;
   const Tallies& T = a.T;
-  const size_t stride = a.prm.slots;
   const uint64_t path = a.first + p.pid;
   const uint32_t flags0 = p.flags;
   uint32_t in_med = p.media & 0xFFFFu, out_med = p.media >> 16;
@@ -532,15 +559,15 @@ __device__ __forceinline__ bool shade_path(const PathArgs& a, Path<F>& p,
         } else {
           real w10[10];
           receiver_weights(in0, in1, in2, kabs, w10);
-          if (!pend_add(a.W.pkey + p.slot, (real*)a.W.pval + p.slot, stride, a.W.npend, p.npk, rkey,
+          const size_t entry = (size_t)p.slot * a.W.npend;
+          if (!pend_add(a.W.pkey + entry, (real*)a.W.pval + entry * 10, a.W.npend, p.npk, rkey,
                         w10)) {
             spill(T.sxr + (size_t)(blockIdx.x & T.mask_x) * T.nsamp * T.nrcv * 40u,
                   (uint64_t)p.samp * S.nrcv * 2u + rkey, w10, &a.C->spills);
           }
-          if (pkey != NONE && !pend_add(a.W.qkey + p.slot, (real*)a.W.qval + p.slot, stride, a.W.npend,
+          if (pkey != NONE && !pend_add(a.W.qkey + entry, (real*)a.W.qval + entry * 10, a.W.npend,
                                         p.nqk, pkey, w10))
-            spill(T.prim + (size_t)(blockIdx.x & T.mask_p) * T.nprim * 40u, pkey, w10,
-                  &a.C->spills);
+            spill_prim(T, pkey, w10, &a.C->spills);
         }
         if (ADJ && a.A.p[p.slot] != NONE) {
           if (pkey != NONE) a.A.s[p.slot].w += a.A.gmap[pkey] * (in0 * kabs);
@@ -606,7 +633,6 @@ template <class F, bool ADJ>
 __device__ __forceinline__ void flush_paths(const PathArgs& a, const Path<F>& p) {
   using real = typename F::real;
   const Tallies& T = a.T;
-  const size_t stride = a.prm.slots;
   const bool done = p.fin == FIN_DONE;
   const double factor = done ? (double)(1u << p.score) : 1.0;
   const bool last = done && p.dkey != NONE;
@@ -640,18 +666,24 @@ __device__ __forceinline__ void flush_paths(const PathArgs& a, const Path<F>& p)
   double* sxr_base = T.sxr + (size_t)(blockIdx.x & T.mask_x) * T.nsamp * T.nrcv * 40u;
   for (int which = 0; which < 2; ++which) {
     const uint32_t n = !done ? 0u : which ? p.nqk : p.npk;
-    const uint32_t* keys = (which ? a.W.qkey : a.W.pkey) + p.slot;
-    const real* vals = (const real*)(which ? a.W.qval : a.W.pval) + p.slot;
+    const size_t entry = (size_t)p.slot * a.W.npend;
+    const uint32_t* keys = (which ? a.W.qkey : a.W.pkey) + entry;
+    const real* vals = (const real*)(which ? a.W.qval : a.W.pval) + entry * 10;
     const uint32_t lkey = !last ? NONE : which ? p.dpkey : p.dkey;
     bool lpend = lkey != NONE;
     for (uint32_t k = 0;; ++k) {
       uint32_t key = NONE;
       real v10[10];
       if (k < n) {
-        key = keys[k * stride];
+        key = keys[k];
         const bool merge = lpend && key == lkey;
-        for (int f = 0; f < 10; ++f)
-          v10[f] = vals[((size_t)k * 10 + f) * stride] + (merge ? dw[f] : real(0));
+        const auto* v = (const WeightPair<real>*)(vals + k * 10);
+#pragma unroll
+        for (int f = 0; f < 5; ++f) {
+          const WeightPair<real> x = v[f];
+          v10[2 * f] = x.a + (merge ? dw[2 * f] : real(0));
+          v10[2 * f + 1] = x.b + (merge ? dw[2 * f + 1] : real(0));
+        }
         if (merge) lpend = false;
       } else if (lpend) {
         key = lkey;

@@ -54,3 +54,28 @@ def test_log_routes_match_atomics(gpu, cells, keys):
     assert len(ref.prim) == keys * 20 and np.count_nonzero(ref.prim) > 1000
     N._same(got, ref, 1.3e-11)
     lib.close()
+
+
+# Paths between two diffuse walls meet more primitives than they hold pending
+# entries for: the rest, logged one by one, against atomics (sums of at most
+# n = 400,000 terms of one sign in two orders: 2 n 2^-53 = 8.9e-11 relative)
+@pytest.mark.parametrize("precision", [0, 1])
+def test_spilled_entries_match_atomics(gpu, precision):
+    wall = S.matte(0.7)
+    obj = S.Object([(S.grid_mesh(4.0, 4.0, 9, 9), wall, wall)])
+    floor = S.Instance(obj, S.IDENTITY, receiver_mask=S.FRONT | S.BACK, per_primitive=1)
+    roof = S.Instance(obj, S.transform(None, (3.0, 0.0, 1.5)), receiver_mask=S.FRONT | S.BACK,
+                      per_primitive=1, sample=0)
+    spec = S.Scene([floor, roof], S.Sun("directional", (0, 0, -1), 1000.0,
+                                        S.Spectrum([1.0], [1.0])), None, name="walls")
+    lib = L.Scene(spec)
+    lib.solve(1000, seed=1)
+    hip, ctx = N._hip(), N._ctx(lib)
+    a = N.SolveArgs(100_000, 2**62, 3, 0, precision, 0, 1, 0)
+    ref, got = N.Out(spec, lib), N.Out(spec, lib)
+    assert hip.ssolh_solve(ctx, C.byref(a)) == 0, hip.ssolh_last_error()
+    assert hip.ssolh_tallies_download(ctx, C.byref(ref.t)) == 0
+    assert hip.ssolh_solve_noalloc(ctx, C.byref(a), C.byref(got.t)) == 0, hip.ssolh_last_error()
+    assert ref.t.pending_spills == got.t.pending_spills > 1000
+    N._same(got, ref, 8.9e-11)
+    lib.close()
