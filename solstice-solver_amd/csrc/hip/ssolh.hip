@@ -46,7 +46,6 @@ namespace {
 
 constexpr int BLOCK = 128;           // threads per block (2 waves)
 constexpr int MAX_STACK = 32;        // traversal stack entries per thread in LDS, largest kernel
-constexpr uint32_t RUN_THROUGH = 1u << 18;  // a launch of at most so many paths runs them to their ends
 constexpr int START_STACK = 20, RESUME_STACK = 32;  // LDS stack entries per lane of the path kernels
 constexpr uint32_t SENTINEL = 0xFFFFFFFFu;
 constexpr uint32_t LEAF = 0x80000000u;
@@ -256,7 +255,7 @@ __device__ __forceinline__ const ssolh_sun& job_sun(const DScene& S, const Solve
   return prm.job_suns ? prm.job_suns[job] : S.sun;
 }
 
-// Adjoint solve (score-function gradients, see k_shade): null grad <=> off.
+// Adjoint solve (score-function gradients, see shade_path): null grad <=> off.
 struct AdjParams {
   double* grad;              // [nparams][3]: d/d aim angle 1, 2, d/d slope error
   const int32_t* inst_param; // [ninstances]: parameter slot of an instance or -1
@@ -2787,9 +2786,14 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
                   k_start<F64, false, false>, k_start<F64, true, false>,
                   k_start<F64, false, true>);
   };
-  // few paths run through, unless their entries could fill the log
+  // Paths that all fit on the chip at once (256 CUs of four SIMDs) run
+  // through, unless their entries could fill the log. A further launch takes
+  // 50 us beside its paths; one round and a third of waves leaves a last
+  // round nearly empty (FP64 cavity of 5e5 paths: 4.75 ms at 2^18, 4.58 at
+  // 3 * 2^16, 4.89 at 2^17).
+  const uint32_t resident = (fp32 ? F32::WAVES : F64::WAVES) * 1024u * 64u;
   auto run_through = [&](uint32_t count) {
-    return count <= RUN_THROUGH && (!c->T.log_cap || count <= c->T.log_cap);
+    return count <= resident && (!c->T.log_cap || count <= c->T.log_cap);
   };
   auto resume = [&](uint32_t count) {
     const uint32_t blocks = (count + BLOCK - 1) / BLOCK;
@@ -2803,7 +2807,7 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
   };
 
   // The realisations first .. first + count - 1 in start-instance order:
-  // drawn keys, then a stable radix sort of (key, index)
+  // drawn keys, grouped, or a stable radix sort of (key, index) (group_pays)
   auto order_starts = [&](uint64_t first, uint32_t count) -> int {
     uint32_t* key = (uint32_t*)c->queue[1].p;
     uint32_t *skey = key + part, *idx = skey + part, *order = idx + part;
