@@ -194,9 +194,12 @@ struct Counters {
   unsigned int iterations, gens;    // generations of rays: of the passes so far, of this one
   unsigned int left;                // length of the list of paths that go on
   unsigned int log_flushes;         // reductions of the per-primitive log
-  unsigned int log_kept;            // records of the reduction under way
   unsigned long long log_over;      // records that found the log full
 };
+
+// Segments of a large per-primitive log, and the distance between their
+// counters (a cache line, in counters)
+constexpr uint32_t LOG_SEGS = 16, LOG_LINE = 16;
 
 // Tallies that every wave updates (global fields, counts) or that few keys
 // share (receivers, sampled instances) are striped: block b adds into
@@ -216,12 +219,15 @@ struct Tallies {
   uint64_t nprim;
   // Log of finished paths' per-primitive entries (prim_add), reduced into
   // `prim` by key (k_prim_reduce): record i is the key log_key[i] and the 10
-  // fields' weights log_val[10 i ..]. log_n counts the records asked for, also
-  // past log_cap (those went to atomics).
+  // fields' weights log_val[10 i ..]. Blocks log to the segment blockIdx &
+  // log_mask, the log_seg records from segment * log_seg on; log_n[segment *
+  // LOG_LINE] counts the records asked for, also past log_seg (those went to
+  // atomics). log_cap: records of all segments, 0 without a log.
   uint32_t* log_key;
   double* log_val;
   unsigned long long* log_n;
   uint64_t log_cap;
+  uint32_t log_seg, log_mask;
 };
 
 struct SolveParams {
@@ -428,10 +434,11 @@ __device__ __forceinline__ void log_record(const Tallies& T, uint64_t pos, uint3
 // whole wave.
 template <typename R>
 __device__ void prim_add(const Tallies& T, bool has, uint32_t key, const R* a, double factor) {
-  const unsigned long long pos = T.log_cap ? wave_count_add(has, T.log_n) : ~0ull;
+  const uint32_t s = blockIdx.x & T.log_mask;
+  const unsigned long long pos = T.log_cap ? wave_count_add(has, T.log_n + s * LOG_LINE) : ~0ull;
   if (!has) return;
-  if (pos < T.log_cap) {
-    log_record(T, pos, key, a, factor);
+  if (pos < T.log_seg) {
+    log_record(T, (uint64_t)s * T.log_seg + pos, key, a, factor);
     return;
   }
   double* pb = T.prim + (size_t)(blockIdx.x & T.mask_p) * T.nprim * 40u + (size_t)key * 20u;
@@ -445,10 +452,6 @@ __device__ void prim_add(const Tallies& T, bool has, uint32_t key, const R* a, d
 
 #include "ssolh_group.hpp"
 
-__global__ void k_iota32(uint32_t* a, uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) a[i] = i;
-}
 
 // -------------------------------------------------------------------------
 // Traversal with the reference hit filter
@@ -1699,7 +1702,7 @@ struct ssolh_context {
   DevBuf plog;
   void* log_sort = nullptr;
   size_t log_sort_bytes = 0;
-  uint32_t *log_skey = nullptr, *log_idx = nullptr, *log_sidx = nullptr;
+  uint32_t *log_ckey = nullptr, *log_skey = nullptr, *log_idx = nullptr, *log_sidx = nullptr;
   uint32_t log_key_bits = 1;
   uint32_t log_cap_test = 0;          // ssolh_test_prim_log's cap (0: the default)
   uint32_t log_flushes = 0;           // the last solve's sorted reductions
@@ -2539,15 +2542,18 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
   // count of the log, the counts of the groupings by start key and by
   // primitive (which each grouping leaves clear), the tallies (striped where
   // many waves meet, see Tallies); beside them the groupings' offsets
-  // (the log's count, which waves add to, on a cache line of its own)
-  constexpr size_t head_bytes = 512;
-  static_assert(sizeof(Counters) <= 256, "head of the cleared buffer");
+  // (the log's counts, which waves add to, on cache lines of their own; a
+  // reduction's record counts)
+  constexpr size_t log_n_at = 256, kept_at = log_n_at + LOG_SEGS * LOG_LINE * 8;
+  constexpr size_t head_bytes = kept_at + 256;
+  static_assert(sizeof(Counters) <= log_n_at && LOG_SEGS <= 64, "head of the cleared buffer");
   const size_t clear_bytes =
       head_bytes + 2 * GROUP_KEYS * sizeof(uint32_t) + (tally_bytes + 15) / 16 * 16;
   if ((r = alloc(c->tallies, clear_bytes + 2 * (GROUP_KEYS + 4) * sizeof(uint32_t)))) return r;
   HIP_TRY(hipMemsetAsync(c->tallies.p, 0, clear_bytes, c->stream));
   Counters* const ctr = (Counters*)c->tallies.p;
-  unsigned long long* const log_n = (unsigned long long*)((char*)c->tallies.p + 256);
+  unsigned long long* const log_n = (unsigned long long*)((char*)c->tallies.p + log_n_at);
+  uint32_t* const log_kept = (uint32_t*)((char*)c->tallies.p + kept_at);
   uint32_t* const group = (uint32_t*)((char*)c->tallies.p + head_bytes);
   uint32_t* const offsets = (uint32_t*)((char*)c->tallies.p + clear_bytes);
   const GroupKeys start_keys{group, offsets, (uint32_t)std::min<uint64_t>(nkeys, UINT32_MAX)};
@@ -2663,12 +2669,22 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
   c->T.log_val = nullptr;
   c->T.log_n = nullptr;
   c->T.log_cap = 0;
+  c->T.log_seg = c->T.log_mask = 0;
+  uint32_t log_segs = 1;
   c->log_flushes = 0;
   c->log_overflowed = 0;
   if (!arena && c->nprim) {
     uint32_t cap = (uint32_t)std::min<uint64_t>(
         std::min<uint64_t>(N, LOG_MAX_RECORDS) * (c->may_pend ? 4 : 1), LOG_MAX_RECORDS);
     if (c->log_cap_test) cap = std::min(cap, c->log_cap_test);
+    // One counter takes 1.6 ns per wave that logs, one wave after the other:
+    // large logs have LOG_SEGS, whose segments (filled evenly, by block) hold
+    // an eighth more than their share (4e6 paths: 1567 us of path kernels
+    // with one counter, 1400 with 16)
+    if (cap >= (1u << 18)) {
+      log_segs = LOG_SEGS;
+      cap = (cap / LOG_SEGS * 9 / 8 + 63) / 64 * 64 * LOG_SEGS;
+    }
     uint32_t bits = 1;
     while (bits < 32 && (uint64_t(1) << bits) < (uint64_t)c->nprim * 2) ++bits;
     group_log = group_pays(cap, (uint64_t)c->nprim * 2);
@@ -2680,7 +2696,7 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
                                                  c->stream));
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
     const size_t k4 = up((size_t)cap * 4);
-    const size_t bytes = 4 * k4 + up((size_t)cap * 80) + up(sort_bytes);
+    const size_t bytes = 5 * k4 + up((size_t)cap * 80) + up(sort_bytes);
     if (alloc(c->plog, bytes)) {
       // no room left beside the path state: every entry takes the atomics
       (void)hipGetLastError();
@@ -2693,19 +2709,22 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
       c->log_skey = (uint32_t*)(q + k4);
       c->log_idx = (uint32_t*)(q + 2 * k4);
       c->log_sidx = (uint32_t*)(q + 3 * k4);
-      c->T.log_val = (double*)(q + 4 * k4);
+      c->log_ckey = (uint32_t*)(q + 4 * k4);
+      c->T.log_val = (double*)(q + 5 * k4);
       c->T.log_n = log_n;
-      c->log_sort = q + 4 * k4 + up((size_t)cap * 80);
+      c->log_sort = q + 5 * k4 + up((size_t)cap * 80);
       c->log_sort_bytes = sort_bytes;
       c->log_key_bits = bits;
       c->T.log_cap = cap;
+      c->T.log_seg = cap / log_segs;
+      c->T.log_mask = log_segs - 1;
     }
   }
   // Sums the logged records into the per-primitive tally and empties the
   // log
   auto log_flush = [&]() -> int {
     if (!c->T.log_cap) return 0;
-    const uint32_t cap = (uint32_t)c->T.log_cap;
+    const uint32_t cap = c->T.log_seg;  // of a segment
     // `shares` waves per key: one round of 64 records each for an even spread
     // of m records, 131,072 waves at most for that. A flux map's peak holds
     // several times the mean: with four rounds its waves run on alone (4e6
@@ -2720,32 +2739,46 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
       return 0;
     };
     if (group_log) {
-      k_group_rank<<<(cap + GROUP_BLOCK - 1) / GROUP_BLOCK, GROUP_THREADS, 0, c->stream>>>(
+      const dim3 rank_grid((cap + GROUP_BLOCK - 1) / GROUP_BLOCK, log_segs);
+      const dim3 place_grid((cap + 255) / 256, log_segs);
+      k_group_rank<<<rank_grid, GROUP_THREADS, 0, c->stream>>>(
           LogKeyOf{c->T.log_key}, c->T.log_n, cap, prim_keys, nullptr, c->log_skey);
       HIP_TRY(hipGetLastError());
-      k_group_scan<<<1, GROUP_THREADS, 0, c->stream>>>(prim_keys, c->T.log_n, cap, &ctr->log_kept, ctr);
+      k_group_scan<<<1, GROUP_THREADS, 0, c->stream>>>(prim_keys, c->T.log_n, log_segs, cap, log_kept,
+                                                       ctr);
       HIP_TRY(hipGetLastError());
-      k_group_place<<<(cap + 255) / 256, 256, 0, c->stream>>>(
-          c->T.log_key, c->log_skey, &ctr->log_kept, 0, prim_keys, c->log_sidx);
+      k_group_place<<<place_grid, 256, 0, c->stream>>>(
+          c->T.log_key, c->log_skey, log_kept, cap, prim_keys, c->log_sidx);
       HIP_TRY(hipGetLastError());
-      return reduce(cap, nullptr);
+      return reduce((uint32_t)c->T.log_cap, nullptr);
     }
-    unsigned long long n = 0;
-    HIP_TRY(hipMemcpyAsync(&n, c->T.log_n, sizeof(n), hipMemcpyDeviceToHost, c->stream));
+    unsigned long long asked[LOG_SEGS * LOG_LINE], n = 0;
+    HIP_TRY(hipMemcpyAsync(asked, c->T.log_n, log_segs * LOG_LINE * sizeof(asked[0]),
+                           hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    const uint32_t m = (uint32_t)std::min<unsigned long long>(n, cap);
+    LogSegments parts{};
+    uint32_t longest = 0;
+    for (uint32_t s = 0; s < log_segs; ++s) {
+      const uint32_t used = (uint32_t)std::min<unsigned long long>(asked[s * LOG_LINE], cap);
+      n += asked[s * LOG_LINE];
+      parts.first[s + 1] = parts.first[s] + used;
+      longest = std::max(longest, used);
+    }
+    const uint32_t m = parts.first[log_segs];
     c->log_overflowed += n - m;
     if (m) {
       ++c->log_flushes;
-      k_iota32<<<(m + 255) / 256, 256, 0, c->stream>>>(c->log_idx, m);
+      const dim3 list_grid((longest + 255) / 256, log_segs);
+      k_log_list<<<list_grid, 256, 0, c->stream>>>(c->T.log_key, cap, parts, c->log_ckey, c->log_idx);
       HIP_TRY(hipGetLastError());
       size_t sb = c->log_sort_bytes;
-      HIP_TRY(hipcub::DeviceRadixSort::SortPairs(c->log_sort, sb, c->T.log_key, c->log_skey,
+      HIP_TRY(hipcub::DeviceRadixSort::SortPairs(c->log_sort, sb, c->log_ckey, c->log_skey,
                                                  c->log_idx, c->log_sidx, (int)m, 0,
                                                  (int)c->log_key_bits, c->stream));
       if (int e = reduce(m, c->log_skey)) return e;
     }
-    if (n) HIP_TRY(hipMemsetAsync(c->T.log_n, 0, sizeof(unsigned long long), c->stream));
+    if (n)
+      HIP_TRY(hipMemsetAsync(c->T.log_n, 0, log_segs * LOG_LINE * sizeof(asked[0]), c->stream));
     return 0;
   };
 
@@ -2821,7 +2854,7 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
       else
         k_group_rank<<<gb, GROUP_THREADS, 0, c->stream>>>(k64, nullptr, count, start_keys, key, skey);
       HIP_TRY(hipGetLastError());
-      k_group_scan<<<1, GROUP_THREADS, 0, c->stream>>>(start_keys, nullptr, 0, nullptr, nullptr);
+      k_group_scan<<<1, GROUP_THREADS, 0, c->stream>>>(start_keys, nullptr, 0, 0, nullptr, nullptr);
       HIP_TRY(hipGetLastError());
       k_group_place<<<gg, 256, 0, c->stream>>>(key, skey, nullptr, count, start_keys, order);
       HIP_TRY(hipGetLastError());
@@ -2869,11 +2902,11 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
         k_queue_list<<<(w + 3) / 4, 256, 0, c->stream>>>(wave_n, w, wave_off, wave_chunk, list);
         HIP_TRY(hipGetLastError());
         uint32_t left = 0;
-        unsigned long long logged = 0;
+        unsigned long long asked[LOG_SEGS * LOG_LINE], logged = 0;
         HIP_TRY(hipMemcpyAsync(&left, &ctr->left, sizeof(left), hipMemcpyDeviceToHost, c->stream));
         if (c->T.log_cap)
-          HIP_TRY(hipMemcpyAsync(&logged, c->T.log_n, sizeof(logged), hipMemcpyDeviceToHost,
-                                 c->stream));
+          HIP_TRY(hipMemcpyAsync(asked, c->T.log_n, log_segs * LOG_LINE * sizeof(asked[0]),
+                                 hipMemcpyDeviceToHost, c->stream));
         HIP_TRY(hipStreamSynchronize(c->stream));
         if (left > going) {
           set_err("ssolh_solve: %u paths go on of %u", left, going);
@@ -2883,7 +2916,9 @@ int run_solve(ssolh_context* c, uint64_t N, uint64_t max_failed, uint64_t key, u
         if (!going) break;
         args.list = list;
         // past half full, the log is summed before it overflows into atomics
-        if (logged && logged >= c->T.log_cap / 2) if ((r = log_flush())) return r;
+        for (uint32_t s = 0; c->T.log_cap && s < log_segs; ++s)
+          logged = std::max(logged, asked[s * LOG_LINE]);
+        if (logged && logged >= c->T.log_seg / 2) if ((r = log_flush())) return r;
       }
       std::swap(from, to);
       args.in = from;
@@ -3286,7 +3321,7 @@ SSOLH_API int ssolh_test_group(ssolh_context* c, uint32_t n, uint32_t nkeys, con
     k_group_rank<<<(n + GROUP_BLOCK - 1) / GROUP_BLOCK, GROUP_THREADS, 0, c->stream>>>(
         LogKeyOf{d_key}, nullptr, n, g, nullptr, d_rank);
     HIP_TRY(hipGetLastError());
-    k_group_scan<<<1, GROUP_THREADS, 0, c->stream>>>(g, nullptr, 0, nullptr, nullptr);
+    k_group_scan<<<1, GROUP_THREADS, 0, c->stream>>>(g, nullptr, 0, 0, nullptr, nullptr);
     HIP_TRY(hipGetLastError());
     k_group_place<<<(n + 255) / 256, 256, 0, c->stream>>>(d_key, d_rank, nullptr, n, g, d_order);
     HIP_TRY(hipGetLastError());

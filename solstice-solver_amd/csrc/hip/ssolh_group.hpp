@@ -40,15 +40,19 @@ struct LogKeyOf {
   __device__ uint32_t operator()(uint32_t i) const { return key[i]; }
 };
 
-// Items 0 .. n - 1, n = min(*n_ptr, cap); key[i] (if not null) and rank[i],
-// its place among the items of its key
+// The items of a log lie in segments of cap places (blockIdx.y), of which
+// those below the segment's count n_ptr[s * LOG_LINE] are in use; without
+// n_ptr they are 0 .. cap - 1. key[i] (if not null) and rank[i], its place
+// among the items of its key
 template <class KeyOf>
 __global__ void __launch_bounds__(GROUP_THREADS)
 k_group_rank(KeyOf key_of, const unsigned long long* n_ptr, uint32_t cap, GroupKeys g,
              uint32_t* __restrict__ key, uint32_t* __restrict__ rank) {
   __shared__ uint32_t hist[GROUP_KEYS];
-  const uint32_t n = n_ptr ? (uint32_t)min(*n_ptr, (unsigned long long)cap) : cap;
-  const uint32_t first = blockIdx.x * GROUP_BLOCK;
+  const uint32_t base = blockIdx.y * cap;
+  const uint32_t used =
+      n_ptr ? (uint32_t)min(n_ptr[blockIdx.y * LOG_LINE], (unsigned long long)cap) : cap;
+  const uint32_t first = base + blockIdx.x * GROUP_BLOCK, n = base + used;
   if (first >= n) return;
   for (uint32_t k = threadIdx.x; k < g.keys; k += GROUP_THREADS) hist[k] = 0;
   __syncthreads();
@@ -77,10 +81,12 @@ k_group_rank(KeyOf key_of, const unsigned long long* n_ptr, uint32_t cap, GroupK
 }
 
 // One block. Also empties the counts for the next grouping and, of a log,
-// its record count (*n_ptr, of which cap were kept): *kept takes the records
-// grouped, C the reduction and the records that found the log full.
+// the record counts of its segments (of which cap each were kept): kept takes
+// the records grouped, C the reduction and the records that found their
+// segment full.
 __global__ void __launch_bounds__(GROUP_THREADS)
-k_group_scan(GroupKeys g, unsigned long long* n_ptr, uint32_t cap, uint32_t* kept, Counters* C) {
+k_group_scan(GroupKeys g, unsigned long long* n_ptr, uint32_t segs, uint32_t cap, uint32_t* kept,
+             Counters* C) {
   __shared__ uint32_t part[GROUP_THREADS];
   constexpr uint32_t per = GROUP_KEYS / GROUP_THREADS;
   const uint32_t tid = threadIdx.x;
@@ -113,21 +119,35 @@ k_group_scan(GroupKeys g, unsigned long long* n_ptr, uint32_t cap, uint32_t* kep
     }
   }
   if (tid == GROUP_THREADS - 1) g.offsets[GROUP_KEYS] = part[tid];
-  if (tid == 0 && n_ptr) {
-    const unsigned long long n = *n_ptr;
+  if (tid < segs && n_ptr) {
+    const unsigned long long n = n_ptr[tid * LOG_LINE];
     const uint32_t m = (uint32_t)min(n, (unsigned long long)cap);
-    *kept = m;
-    *n_ptr = 0;
-    C->log_over += n - m;
-    if (m) ++C->log_flushes;
+    kept[tid] = m;
+    n_ptr[tid * LOG_LINE] = 0;
+    if (n > m) atomicAdd(&C->log_over, n - m);
   }
+  if (tid == 0 && n_ptr && part[GROUP_THREADS - 1]) ++C->log_flushes;
 }
 
 __global__ void __launch_bounds__(256)
 k_group_place(const uint32_t* __restrict__ key, const uint32_t* __restrict__ rank,
               const uint32_t* kept, uint32_t n, GroupKeys g, uint32_t* __restrict__ order) {
-  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  if (i < (kept ? *kept : n)) order[g.offsets[key[i]] + rank[i]] = i;
+  const uint32_t j = blockIdx.x * 256u + threadIdx.x, i = blockIdx.y * n + j;
+  if (j < (kept ? kept[blockIdx.y] : n)) order[g.offsets[key[i]] + rank[i]] = i;
+}
+
+// The keys and indices of a log's records side by side, for the radix sort:
+// segment s (cap places, first[s + 1] - first[s] of them in use) from first[s]
+struct LogSegments {
+  uint32_t first[LOG_SEGS + 1];
+};
+__global__ void __launch_bounds__(256)
+k_log_list(const uint32_t* __restrict__ log_key, uint32_t cap, LogSegments s,
+           uint32_t* __restrict__ key, uint32_t* __restrict__ idx) {
+  const uint32_t j = blockIdx.x * 256u + threadIdx.x, to = s.first[blockIdx.y] + j;
+  if (to >= s.first[blockIdx.y + 1]) return;
+  key[to] = log_key[blockIdx.y * cap + j];
+  idx[to] = blockIdx.y * cap + j;
 }
 
 // First of the sorted keys skey[0 .. m) that is not below k: the wave probes

@@ -344,10 +344,11 @@ __device__ void spill(double* base, uint64_t key, const R* w, unsigned long long
 template <typename R>
 __device__ void spill_prim(const Tallies& T, uint32_t key, const R* w, unsigned long long* spills) {
   if (T.log_cap) {
-    const unsigned long long pos = atomicAdd(T.log_n, 1ull);
-    if (pos < T.log_cap) {
+    const uint32_t s = blockIdx.x & T.log_mask;
+    const unsigned long long pos = atomicAdd(T.log_n + s * LOG_LINE, 1ull);
+    if (pos < T.log_seg) {
       atomicAdd(spills, 1ull);
-      log_record(T, pos, key, w, 1.0);
+      log_record(T, (uint64_t)s * T.log_seg + pos, key, w, 1.0);
       return;
     }
   }
