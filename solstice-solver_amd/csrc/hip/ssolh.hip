@@ -2335,7 +2335,6 @@ SSOLH_API int ssolh_render(ssolh_context* c, const struct ssolh_render_args* a, 
     rp.first = first;
     rp.count = (uint32_t)std::min<uint64_t>(total - first, batch);
     const uint32_t blocks = (rp.count + BLOCK - 1) / BLOCK;
-    HIP_TRY(hipMemsetAsync(cnt, 0, 16, c->stream));
     k_render_start<<<blocks, BLOCK, 0, c->stream>>>(c->scn, rp, st, rays, lists[0], cnt);
     HIP_TRY(hipGetLastError());
     int cur = 0;

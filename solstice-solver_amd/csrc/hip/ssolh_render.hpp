@@ -99,25 +99,32 @@ __device__ double render_bsdf_sample(const ssolh_material& m, double eta_out, do
   return bsdf_sample(m, eta_out, eta_in, slab_eta, slab_abs, wi, n, rng, wo, lobe);
 }
 
-// Appends `slot` to the work list (one atomic per wave)
-__device__ __forceinline__ void render_push(bool has, uint32_t slot, uint32_t* list,
+// Appends sample s's bounce ray (slot 2s) and sun ray (2s + 1) to the work
+// list, with one atomic per wave: the waves' adds to the count follow one
+// another, 11 ns each.
+__device__ __forceinline__ void render_push(bool bounce, bool sun, uint32_t s, uint32_t* list,
                                             unsigned* count) {
-  const uint64_t mask = __ballot(has);
-  if (!mask) return;
-  const int leader = __ffsll((unsigned long long)mask) - 1;
+  const uint64_t mb = __ballot(bounce), ms = __ballot(sun);
+  if (!(mb | ms)) return;
+  const uint64_t below = (1ull << lane_id()) - 1ull;
+  const unsigned nb = (unsigned)__popcll(mb);
   unsigned base = 0;
-  if ((int)lane_id() == leader) base = atomicAdd(count, (unsigned)__popcll(mask));
-  base = __shfl(base, leader, 64);
-  if (has) list[base + __popcll(mask & ((1ull << lane_id()) - 1ull))] = slot;
+  if (lane_id() == 0) base = atomicAdd(count, nb + (unsigned)__popcll(ms));
+  base = __shfl(base, 0, 64);
+  if (bounce) list[base + __popcll(mb & below)] = 2 * s;
+  if (sun) list[base + nb + __popcll(ms & below)] = 2 * s + 1;
 }
 
-// Camera rays of the batch's samples (slot 2s; slot 2s + 1 is the sun ray)
+// Camera rays of the batch's samples (slot 2s; slot 2s + 1 is the sun ray).
+// Every sample has one, so the list needs no counting (an atomic per wave
+// took 336 us for 1.8M samples; 63 without). Bound by its stores.
 __global__ void __launch_bounds__(BLOCK)
 k_render_start(DScene S, RenderParams rp, RenderState* __restrict__ st, RayRec* __restrict__ rays,
                uint32_t* list, unsigned* count) {
   const uint32_t s = blockIdx.x * BLOCK + threadIdx.x;
-  const bool live = s < rp.count;
-  if (live) {
+  if (s == 0) *count = rp.count;
+  if (s < rp.count) {
+    list[s] = 2 * s;
     const uint64_t g = rp.first + s;
     const uint32_t pixel = (uint32_t)(g / rp.spp), k = (uint32_t)(g % rp.spp);
     const uint32_t px = pixel % rp.width, py = pixel / rp.width;
@@ -157,7 +164,6 @@ k_render_start(DScene S, RenderParams rp, RenderState* __restrict__ st, RayRec* 
     x.block = rng.block;
     st[s] = x;
   }
-  render_push(live, 2 * s, list, count);
 }
 
 // One bounce of every live sample: the sun ray's result, then the hit of
@@ -271,6 +277,5 @@ k_render_shade(DScene S, RenderParams rp, RenderState* __restrict__ st,
     }
     st[s] = x;
   }
-  render_push(emit_bounce, 2 * s, list, count);
-  render_push(emit_sun, 2 * s + 1, list, count);
+  render_push(emit_bounce, emit_sun, s, list, count);
 }
