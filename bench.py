@@ -119,7 +119,8 @@ def load_traffic(kernel, workload):
 
 
 def other_forms(spec, B, ttt_batch, args):
-    """The FP32 form and the graph-captured FP64 form on the same field:
+    """The FP32 form and both forms with graph_iterations set (which changes
+    nothing) on the same field:
     Mpaths/s, time to 0.1% rel. SE on absorbed, and the FP32 estimate's
     difference from an FP64 run of the same size (in combined SE)."""
     import ssol_ctypes as L
@@ -153,8 +154,7 @@ def other_forms(spec, B, ttt_batch, args):
 def sweep(n_suns=512, log_min=5.0, log_max=7.0, seq_suns=64, graph_iterations=16):
     """The 100-paraboloid field under n_suns sun positions with seeded
     log-uniform realisation counts: one batched solve driven by the host
-    loop, the same batch with graph_iterations wavefront iterations per HIP
-    graph launch and, for comparison, the first seq_suns suns as separate
+    loop, the same batch with graph_iterations set and, for comparison, the first seq_suns suns as separate
     ssol_solve calls on the same scene through the public API (each sun
     change re-flattens the scene, as any caller's per-sun solve would)."""
     import ctypes as C
@@ -349,7 +349,7 @@ def main(argv=None):
     ap.add_argument("--precision", choices=("fp64", "fp32"), default="fp64")
     ap.add_argument("--path-slots", type=int, default=0)
     ap.add_argument("--graph", type=int, default=0,
-                    help="wavefront iterations per HIP graph launch (0: host-driven)")
+                    help="graph_iterations of the device (changes nothing)")
     ap.add_argument("--cpu-seconds", type=float, default=15.0)
     ap.add_argument("--cpu-ttt-seconds", type=float, default=40.0,
                     help="bound on the CPU time-to-0.1%% run (0: skip it)")
@@ -357,7 +357,7 @@ def main(argv=None):
     ap.add_argument("--no-copy", action="store_true", help="skip the copy-bandwidth yardstick")
     ap.add_argument("--no-ttt", action="store_true", help="skip the time-to-0.1%% run")
     ap.add_argument("--no-forms", action="store_true",
-                    help="skip the FP32 / graph-captured forms, the sweep and the adjoint")
+                    help="skip the other forms, the sweep and the adjoint")
     args = ap.parse_args(argv)
 
     if args.gpus != 1:
@@ -409,7 +409,8 @@ def main(argv=None):
     # roofline of the path kernels, from in-stream HIP events
     fp32 = args.precision == "fp32"
     kernel, ms = ("k_path32" if fp32 else "k_path"), trace_ms
-    per_seg = BYTES_PATH_FP32 if fp32 else BYTES_PATH_FP64
+    # a path's first ray reads no record and its last writes none
+    per_seg = (BYTES_PATH_FP32 if fp32 else BYTES_PATH_FP64) * (segs - B * args.steps) / segs
     achieved = per_seg * segs / (ms * 1e-3) / 1e9
     seg_per_launch = segs / iters
     tr = load_traffic(kernel, workload + ("_fp32" if fp32 else ""))
@@ -417,7 +418,7 @@ def main(argv=None):
     roofline = {"bound": "hbm", "kernel": kernel, "achieved": round(achieved, 2),
                 "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 5),
                 "traffic": traffic, "algorithmic_bytes_per_launch": round(per_seg * seg_per_launch),
-                "bytes_per_segment": per_seg, "avg_launch_ms": round(ms / iters, 4),
+                "bytes_per_segment": round(per_seg, 1), "avg_launch_ms": round(ms / iters, 4),
                 "segments_per_path": round(segs / (B * args.steps), 4),
                 "trace_ms_per_step": round(trace_ms / args.steps, 3),
                 "shade_ms_per_step": round(shade_ms / args.steps, 3)}

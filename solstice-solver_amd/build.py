@@ -28,8 +28,9 @@ HIPCC_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
                # no machine-level hoisting of loop invariants: it lifts the
                # FP64 polynomial and Threefry constants of the path kernels
                # out of their loops and keeps them live across them, which
-               # spills (k_shade 108 -> 60 bytes/lane of scratch, k_generate
-               # 92 -> 0, the looping graph-captured forms 388 -> 72)
+               # spills (bytes per lane without and with the flag, FP64:
+               # k_start 112 -> 0, k_resume 60 -> 0, to the paths' ends
+               # 308 -> 140; FP32: 176 -> 16, 80 -> 44, 164 -> 116)
                "-mllvm", "-disable-machine-licm"]
 
 

@@ -9,10 +9,10 @@
 // place and follows each to its end. Form: the FP64 form F64 or the FP32 form
 // F32 (ssolh_fp32.hpp).
 
-// What bounds them: vector issue and the latency of the traversal's node
-// loads, a third to a half of the cycles each (rocprofv3: k_start 40 % VALU
-// busy, the passes after it 51-54 %, texture addresser 60 %); HBM traffic is
-// 0.9 TB/s. Waves per SIMD, measured on the 10k-heliostat field (3e7 FP64,
+// What bounds them: vector issue and the traversal's node loads (rocprofv3,
+// 1e8 FP64 paths: k_start 73 % VALU busy with 78 % of the lanes active, the
+// passes after it 57-63 % with 45-65 %, texture addresser 47-61 %); HBM
+// traffic is 1.7 TB/s. Waves per SIMD, measured on the 10k-heliostat field (3e7 FP64,
 // 1e7 FP32 paths): FP64 16.3 ms at three (no spills), 18.0 at four (60 to 132
 // bytes per lane spilled); FP32 5.3 ms at four, 5.7 at three. Separate
 // generate, trace, shade and compaction launches, which the path kernels
